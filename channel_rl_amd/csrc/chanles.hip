@@ -108,7 +108,8 @@ struct chan_ctx {
     void* dsm[13] = {};
     const void* rcp[2][6] = {};  // reciprocal spacings [double, float][dx, dy, dz, dxg, dyg, dzg]
     double* part = nullptr;
-    int nblk_dsm = 0, nblk_red = 0, dsm_kchunk = 16, dsm_shape = 0;
+    int nblk_red = 0, dsm_shape = 0;
+    DsmPlan dsm_run{};  // how dsm_shape runs on this channel alone
     double* ratio = nullptr;
     double* alpha = nullptr;
     double* stage = nullptr;
@@ -119,7 +120,6 @@ struct chan_ctx {
     // the same steps with compute_dt folded into substep 1 (dt_fused)
     hipGraphExec_t graph_dt[3] = {nullptr, nullptr, nullptr};
     double* dtpart = nullptr;  // the DSM pass's compute_dt maxima, [3][blocks]
-    int nblk_dt = 0;
     // substeps 1 and 2 of a step leave the dynamic model's pass B to the RHS
     // kernel (DsmBufs::ntab): its row coefficients, [2][nyg] of the bulk type
     void* ntab = nullptr;
@@ -270,9 +270,9 @@ DsmBufs<T> dsm_bufs(chan_ctx* c)
     b.smag = (T*)c->dsm[9];
     b.part = c->part;
     b.ratio = c->ratio;
-    b.nblk = c->nblk_dsm;
-    b.kchunk = c->dsm_kchunk;
-    b.shape = c->dsm_shape;
+    b.nblk = c->dsm_run.nblk;
+    b.kchunk = c->dsm_run.kchunk;
+    b.tile = c->dsm_run.tile;
     const int pi = sizeof(T) == sizeof(double) ? 0 : 1;
     b.rdx = (const T*)c->rcp[pi][0]; b.rdy = (const T*)c->rcp[pi][1]; b.rdz = (const T*)c->rcp[pi][2];
     b.rdxg = (const T*)c->rcp[pi][3]; b.rdyg = (const T*)c->rcp[pi][4]; b.rdzg = (const T*)c->rcp[pi][5];
@@ -280,7 +280,7 @@ DsmBufs<T> dsm_bufs(chan_ctx* c)
     b.ntab = nullptr;    // set by the substeps that defer pass B
     b.xg = c->md.xg; b.yg = c->md.yg; b.zg = c->md.zg;
     b.mins3 = c->mins3;
-    b.nblk_dt = c->nblk_dt;
+    b.nblk_dt = c->dsm_run.blocks;
     return b;
 }
 
@@ -469,19 +469,11 @@ int net_order(chan_ctx* c)
     return CHAN_OK;
 }
 
-// the DSM pass A tile shape q with its z chunk and partial-sum block count
+// the DSM pass A tile shape q and how it runs on this channel
 void set_dsm_shape(chan_ctx* c, int q)
 {
     c->dsm_shape = q;
-    if (c->prec == CHAN_FP64) {
-        c->dsm_kchunk = dsm_fused_kchunk<double>(c->d, c->device, q);
-        c->nblk_dsm = dsm_fused_nblk<double>(c->d, c->dsm_kchunk, q);
-        c->nblk_dt = dsm_fused_blocks<double>(c->d, c->dsm_kchunk, q);
-    } else {
-        c->dsm_kchunk = dsm_fused_kchunk<float>(c->d, c->device, q);
-        c->nblk_dsm = dsm_fused_nblk<float>(c->d, c->dsm_kchunk, q);
-        c->nblk_dt = dsm_fused_blocks<float>(c->d, c->dsm_kchunk, q);
-    }
+    c->dsm_run = c->prec == CHAN_FP64 ? dsm_plan<double>(c->d, c->device, q) : dsm_plan<float>(c->d, c->device, q);
 }
 
 // compute_dt folded into the step's first DSM pass: the dynamic Smagorinsky
@@ -705,8 +697,8 @@ int chan_create(const chan_config* cfg, chan_ctx** out)
     size_t nblk_max = 0, nblk_dt_max = 0;
     for (int q = dsm_shape_count() - 1; q >= 0; q--) {
         set_dsm_shape(c, q);
-        nblk_max = std::max(nblk_max, (size_t)c->nblk_dsm);
-        nblk_dt_max = std::max(nblk_dt_max, (size_t)c->nblk_dt);
+        nblk_max = std::max(nblk_max, (size_t)c->dsm_run.nblk);
+        nblk_dt_max = std::max(nblk_dt_max, (size_t)c->dsm_run.blocks);
     }
     if (c->LES_model == 3) nblk_dt_max = amd_blocks(d);
     if ((c->LES_model == 2 || c->LES_model == 3) &&
@@ -1371,7 +1363,7 @@ void tune_dsm(chan_ctx* c)
 {
     T** I = (T**)c->state[c->cur];
     DsmBufs<T> b = dsm_bufs<T>(c);
-    launch_dsm_fused<T>(I[0], I[1], I[2], metric<T>(c), c->d, b, c->stream);
+    run_dsm_fused<T>(DsmArgs<T>{I[0], I[1], I[2], b}, nullptr, 1, c->d, b.kchunk, b.tile, c->stream);
 }
 int tune_launch(chan_ctx* c, int kernel)
 {
@@ -1572,9 +1564,7 @@ bool same_group(const chan_ctx* a, const chan_ctx* b)
 {
     return a->prec == b->prec && a->d.nx == b->d.nx && a->d.ny == b->d.ny && a->d.nz == b->d.nz &&
            a->LES_model == 2 && b->LES_model == 2 && a->wall_mode == b->wall_mode && a->x_mass_cte == b->x_mass_cte &&
-           a->rhs_shape == b->rhs_shape && a->dsm_shape == b->dsm_shape && a->dsm_kchunk == b->dsm_kchunk &&
-           a->nblk_dsm == b->nblk_dsm &&
-           a->nblk_red == b->nblk_red && a->pb.bx == b->pb.bx && a->pb.bz == b->pb.bz;
+           a->rhs_shape == b->rhs_shape && a->dsm_run.tile == b->dsm_run.tile && a->nblk_red == b->nblk_red && a->pb.bx == b->pb.bx && a->pb.bz == b->pb.bz;
 }
 
 template <typename T>
@@ -1653,8 +1643,9 @@ int enqueue_group_step(chan_ensemble* e, const std::vector<int>& idx, TabSink& s
             const DsmRatioArgs* tr = sink.put(r);
             const DsmNutArgs<T>* tv = sink.put(v);
             if (sink.launch) {
-                run_dsm_fused<T>(a[0], ta, n, d, c0->dsm_kchunk, c0->dsm_shape, s);
-                run_dsm_ratio(r[0], tr, n, d, c0->nblk_dsm, s);
+                const DsmPlan pl = dsm_plan<T>(d, e->device, c0->dsm_run.tile, n);
+                run_dsm_fused<T>(a[0], ta, n, d, pl.kchunk, pl.tile, s);
+                run_dsm_ratio(r[0], tr, n, d, pl.nblk, s);
                 if (defer) run_dsm_edges<T>(v[0], tv, n, d, s);
                 else run_dsm_nut<T>(v[0], tv, n, d, 1, s);
             }

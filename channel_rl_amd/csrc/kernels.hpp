@@ -16,12 +16,12 @@ struct EqAlphaArgs;
 // Work buffers of the dynamic Smagorinsky model (box layout, type T).
 template <typename T>
 struct DsmBufs {
-    T* smag;       // |S| (box layout)
+    T* smag;       // |S| (box layout, rows 2..nyg-1 with their periodic images)
     double* part;  // per-block partial sums: [nyg][2][nblk]
     double* ratio; // <LM>/<MM> per row (index j-1); also LM, MM at +nyg, +2nyg
     int nblk;      // partial-sum blocks per row
     int kchunk;    // z planes per block of the fused pass A
-    int shape;     // tile shape of the fused pass A (dsm_shape_count)
+    int tile;      // tile of the fused pass A (DsmPlan)
     // reciprocal spacings, 1-based: 1/(x(i)-x(i-1)), 1/(xg(i)-xg(i-1)), ...
     const T *rdx, *rdy, *rdz, *rdxg, *rdyg, *rdzg;
     // compute_dt's maxima over the pass's output cells, when dtpart is set:
@@ -35,8 +35,7 @@ struct DsmBufs {
     // is left to the consumer of nu_t: the ratio launch writes per row j the
     // coefficients (A, B) at ntab[c*nyg + j-1] with nu_t = max(A v, B) for
     // the value v that smag then holds at a cell, and a small kernel puts the
-    // wall model's nu_t into smag's wall rows and completes the periodic
-    // images of the others; nu_t itself is not written
+    // wall model's nu_t into smag's wall rows; nu_t itself is not written
     T* ntab;
 };
 
@@ -78,19 +77,23 @@ void launch_amd(const T* U, const T* V, const T* W, T* nut, const Metric<T>& m, 
                 const double* mins3 = nullptr);
 int amd_blocks(const Dims& d);
 
-// fused pass A of the dynamic Smagorinsky model (dsm_fused.hip): z-chunk
-// length for this grid and device, and the partial-sum blocks per row it gives
+// fused pass A of the dynamic Smagorinsky model (dsm_fused.hip in FP64,
+// dsm_fp32.hip in FP32): how a tile shape runs for nmem channels in one launch.
+// FP64: shape 0 is picked by the grid; neither nblk nor the result depends on
+// the chunk.  FP32: the chunk is the channel's own whatever nmem.
+struct DsmPlan {
+    int tile;    // the tile in use
+    int kchunk;  // z planes per block
+    int nblk;    // partial sums per row
+    int blocks;  // blocks of one channel
+};
 template <typename T>
-int dsm_fused_kchunk(const Dims& d, int device, int shape);
-template <typename T>
-int dsm_fused_nblk(const Dims& d, int kchunk, int shape);
-template <typename T>
-int dsm_fused_blocks(const Dims& d, int kchunk, int shape);
+DsmPlan dsm_plan(const Dims& d, int device, int shape, int nmem = 1);
+template <>
+DsmPlan dsm_plan<double>(const Dims& d, int device, int shape, int nmem);
+template <>
+DsmPlan dsm_plan<float>(const Dims& d, int device, int shape, int nmem);
 int dsm_shape_count();
-template <typename T>
-void launch_dsm_fused(const T* U, const T* V, const T* W, const Metric<T>& m, const Dims& d, DsmBufs<T>& b,
-                      hipStream_t s);
-
 template <typename T>
 void launch_wall_model(const T* U, T* nut, const double* alpha_x, const Metric<T>& m, const Dims& d, T nu,
                        const Scalars* sc, hipStream_t s);
@@ -210,8 +213,12 @@ void run_mass_flow_correct(const MassArgs<T>& one, const MassArgs<T>* tab, int n
 template <typename T>
 void run_dt(const DtArgs<T>& one, const DtArgs<T>* tab, int nmem, const Dims& d, int nblk, hipStream_t s);
 template <typename T>
-void run_dsm_fused(const DsmArgs<T>& one, const DsmArgs<T>* tab, int nmem, const Dims& d, int kchunk, int shape,
+void run_dsm_fused(const DsmArgs<T>& one, const DsmArgs<T>* tab, int nmem, const Dims& d, int kchunk, int tile,
                    hipStream_t s);
+template <>
+void run_dsm_fused<double>(const DsmArgs<double>&, const DsmArgs<double>*, int, const Dims&, int, int, hipStream_t);
+template <>
+void run_dsm_fused<float>(const DsmArgs<float>&, const DsmArgs<float>*, int, const Dims&, int, int, hipStream_t);
 template <typename T>
 void run_rhs_rk(const RhsArgs<T>& one, const RhsArgs<T>* tab, int nmem, const Dims& d, int mode, double c1,
                 double c2, int shape, hipStream_t s);

@@ -210,13 +210,9 @@ __global__ void __launch_bounds__(256) k_dsm_nut(DsmNutArgs<T> one, const DsmNut
     }
 }
 
-// The rest of a deferred pass B (DsmBufs::ntab): in the |S| box itself,
-// which pass A filled on the unique cells of rows 2..nyg-1,
-//   the wall model's nu_t on rows 1, 2, nyg-1, nyg (the values k_dsm_nut
-//   writes there with fuse_wm), every cell with its periodic images; then
-//   the x image columns 1, nxg-1, nxg and z image planes 1, nzg-1, nzg of
-//   rows 3..nyg-2, from their unique cells.
-// No thread reads a cell that another one writes.
+// The rest of a deferred pass B (DsmBufs::ntab): the wall model's nu_t on rows
+// 1, 2, nyg-1, nyg of the |S| box (the values k_dsm_nut writes there with
+// fuse_wm), every cell with its periodic images; pass A filled the other rows.
 template <typename T>
 __global__ void __launch_bounds__(256) k_dsm_edges(DsmNutArgs<T> one, const DsmNutArgs<T>* tab, Dims d)
 {
@@ -225,40 +221,20 @@ __global__ void __launch_bounds__(256) k_dsm_edges(DsmNutArgs<T> one, const DsmN
     T* S = a.nut;  // the |S| box (the launcher passes it as nut)
     const long q = (long)g.x * blockDim.x + threadIdx.x;
     const int nxz = d.nxg * d.nzg;
-    if (q < 2L * nxz) {
-        const int side = (int)(q / nxz), r = (int)(q - (long)side * nxz);
-        const int k = r / d.nxg + 1, i = r - (k - 1) * d.nxg + 1;
-        const T v = wm_nut_at<T>(a.U, a.alpha, a.m, d, a.nu, img_centre(i, d.nxg), k, side, a.sc);
-        const int j0 = side == 0 ? 1 : d.nyg - 1;
-        S[at(d, i, j0, k)] = v;
-        S[at(d, i, j0 + 1, k)] = v;
-        return;
-    }
-    const int npos = 3 * d.nzg + 3 * (d.nxg - 3);
-    const long t = q - 2L * nxz;
-    if (t >= (long)npos * (d.nyg - 4)) return;
-    const int row = (int)(t / npos), pos = (int)(t - (long)row * npos);
-    const int j = row + 3;
-    int i, k;
-    if (pos < 3 * d.nzg) {
-        const int c = pos / d.nzg;
-        i = c == 0 ? 1 : d.nxg - 2 + c;
-        k = pos - c * d.nzg + 1;
-    } else {
-        const int p2 = pos - 3 * d.nzg, c = p2 / (d.nxg - 3);
-        k = c == 0 ? 1 : d.nzg - 2 + c;
-        i = p2 - c * (d.nxg - 3) + 2;
-    }
-    S[at(d, i, j, k)] = S[at(d, img_centre(i, d.nxg), j, img_centre(k, d.nzg))];
+    if (q >= 2L * nxz) return;
+    const int side = (int)(q / nxz), r = (int)(q - (long)side * nxz);
+    const int k = r / d.nxg + 1, i = r - (k - 1) * d.nxg + 1;
+    const T v = wm_nut_at<T>(a.U, a.alpha, a.m, d, a.nu, img_centre(i, d.nxg), k, side, a.sc);
+    const int j0 = side == 0 ? 1 : d.nyg - 1;
+    S[at(d, i, j0, k)] = v;
+    S[at(d, i, j0 + 1, k)] = v;
 }
 
 template <typename T>
 void run_dsm_edges(const DsmNutArgs<T>& one, const DsmNutArgs<T>* tab, int nmem, const Dims& d, hipStream_t s)
 {
-    const int npos = 3 * d.nzg + 3 * (d.nxg - 3);
-    const long n = 2L * d.nxg * d.nzg + (long)npos * (d.nyg - 4);
     PROF_BEGIN("k_dsm_edges", s);
-    k_dsm_edges<T><<<dim3(cdiv(n, 256), 1, nmem), 256, 0, s>>>(one, tab, d);
+    k_dsm_edges<T><<<dim3(cdiv(2L * d.nxg * d.nzg, 256), 1, nmem), 256, 0, s>>>(one, tab, d);
     PROF_END(s);
 }
 
@@ -286,7 +262,7 @@ void launch_dsm(const T* U, const T* V, const T* W, T* nut, const Metric<T>& m, 
                 int dirichlet, int fuse_wm, const double* alpha_x, T nu, const Scalars* sc, hipStream_t s,
                 const EqAlphaArgs<T>* eq)
 {
-    launch_dsm_fused<T>(U, V, W, m, d, b, s);
+    run_dsm_fused<T>(DsmArgs<T>{U, V, W, b}, nullptr, 1, d, b.kchunk, b.tile, s);
     DsmRatioArgs ra{b.part, b.ratio, b.dtpart, b.nblk_dt, const_cast<Scalars*>(sc), b.dtpart ? b.mins3 : nullptr};
     ra.fp32 = sizeof(T) == 4;
     if (eq) {
