@@ -372,28 +372,78 @@ __global__ void __launch_bounds__(TX* TY)
 }
 
 // Tile shapes (x cells, y cells) and z-chunk lengths the launcher offers;
-// chan_autotune times them on the channel at hand.  kchunk 0: the chunk that
-// fills the last round of blocks on this grid and device
-// (round_filling_chunk with the kernel's occupancy), counting the tiles of
-// every member of a grouped launch (each cell is computed once whatever the
-// chunk, so the results do not depend on it).
+// chan_autotune times them on the channel at hand.  kchunk 0: the chunk of
+// least modelled time on this grid and device (rhs_pick); tx 0: the tile too.
+// Each cell is computed once whatever the tile and chunk, so the results do
+// not depend on them.
 struct RhsShape { int tx, ty, kchunk; };
 static const RhsShape kRhsShapes[] = {
-    {64, 4, 16}, {64, 4, 8}, {64, 8, 8}, {64, 8, 16}, {32, 8, 8}, {32, 8, 16}, {64, 4, 32}, {64, 8, 32},
+    {0, 0, 0},   {64, 4, 8}, {64, 8, 8}, {64, 8, 16}, {32, 8, 8}, {32, 8, 16}, {64, 4, 32}, {64, 8, 32},
     {64, 4, 0},  {32, 8, 0}, {64, 8, 0},
 };
 
-template <typename T, int TX, int TY>
-int rhs_round_chunk(int ni, int nj, int nk, int nmem)
+// Modelled time of a launch in planes of a lone block (3.0 us in FP64, 2.6 in
+// FP32): blocks run in rounds of per_cu x ncu, a round costs the pre-roll of
+// three planes (1.6) plus its planes, each dearer by s per further block on
+// the CU.  With per_cu blocks everywhere a plane takes 1.7 (FP64, 3 blocks)
+// or 1.5 (FP32, 4), where the memory system is the bound, so a grid with few
+// tiles wants chunks so short that every CU has a block, a large one the
+// chunk that fills its last round.  Chunks beyond 16 planes only lose (a
+// tile's halo rows leave L2 before the neighbour's march reads them:
+// 384x192x384 FP64 673 us with 12, 684 with 16, 708 with 24).
+// Measured with this rule against 64x4 tiles in 16-plane chunks (us, FP64 /
+// FP32): 32x32x32 7.9 / 7.1 against 54 / 47, 128x40x64 16.8 / 11.9 against
+// 53 / 46, 96x64x96 23.4 / 15.7 against 54 / 47, 120x58x90 26.6 / 18.0
+// against 54 / 46, 128x96x128 46.9 / 31.0 against 65 / 48, 192x96x192 98 / 62
+// against 115 / 66, 384x192x384 684 / 377 against 684 / 380.
+struct RhsTile { int tx, ty, per_cu; double s; };
+struct RhsPick { int tx, ty, kc; double cost; };
+static RhsPick rhs_pick(const RhsTile& t, int ni, int nj, int nk, int nmem, int ncu)
 {
-    int per_cu = 0, ncu = 0, dev = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_rhs_rk<T, TX, TY, 2, false>, TX * TY, 0) != hipSuccess ||
-        per_cu < 1)
-        per_cu = 1;
+    const double pre = 1.6;
+    const long tiles = (long)cdiv(ni, t.tx) * cdiv(nj, t.ty) * nmem, slots = (long)t.per_cu * ncu;
+    RhsPick best{t.tx, t.ty, 1, 0.0};
+    for (int kc = 1; kc <= std::min(nk, 16); kc++) {
+        const long blocks = tiles * cdiv(nk, kc), rest = blocks % slots;
+        double cost = (double)(blocks / slots) * (pre + kc * (1.0 + t.s * (t.per_cu - 1)));
+        if (rest) cost += pre + kc * (1.0 + t.s * (cdiv(rest, ncu) - 1));
+        if (kc == 1 || cost < best.cost) {
+            best.cost = cost;
+            best.kc = kc;
+        }
+    }
+    return best;
+}
+
+template <typename T, int TX, int TY>
+RhsTile rhs_tile()
+{
+    // resident blocks per CU: a property of the kernel, the same on every gfx950
+    static const int per_cu = [] {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_rhs_rk<T, TX, TY, 2, false>, TX * TY, 0) != hipSuccess)
+            n = 1;
+        return std::max(n, 1);
+    }();
+    return RhsTile{TX, TY, per_cu, sizeof(T) == 8 ? 0.35 : 0.17};
+}
+
+// tile and chunk of a launch, counting the tiles of every member of a group
+template <typename T>
+RhsPick rhs_plan(const RhsShape& sh, int ni, int nj, int nk, int nmem)
+{
+    if (sh.kchunk > 0) return RhsPick{sh.tx, sh.ty, std::min(RHS_KMAX, sh.kchunk), 0.0};
+    int ncu = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
         ncu = 1;
-    return round_filling_chunk((long)cdiv(ni, TX) * cdiv(nj, TY) * nmem, nk, (long)per_cu * ncu, 6, 32);
+    if (sh.tx == 64 && sh.ty == 8) return rhs_pick(rhs_tile<T, 64, 8>(), ni, nj, nk, nmem, ncu);
+    const RhsPick a = rhs_pick(rhs_tile<T, 64, 4>(), ni, nj, nk, nmem, ncu);
+    const RhsPick b = rhs_pick(rhs_tile<T, 32, 8>(), ni, nj, nk, nmem, ncu);
+    if (sh.tx) return sh.tx == 64 ? a : b;
+    // 32 columns only where they save work: at the same cost the longer rows
+    // of 64 read fewer halo lines (128x96x128 FP64: 46.9 us against 50.2)
+    return b.cost < a.cost ? b : a;
 }
 int rhs_shape_count() { return (int)(sizeof(kRhsShapes) / sizeof(kRhsShapes[0])); }
 
@@ -404,7 +454,9 @@ void run_rhs_rk(const RhsArgs<T>& one, const RhsArgs<T>* tab, int nmem, const Di
     const RhsShape sh = kRhsShapes[(shape >= 0 && shape < rhs_shape_count()) ? shape : 0];
     const int ni = (mode == 0 ? d.nxg - 1 : d.nxg - 2) - 1;
     const int nk = (mode == 0 ? d.nzg - 1 : d.nzg - 2) - 1;
-    dim3 blk(sh.tx, sh.ty, 1);
+    const RhsPick pk = rhs_plan<T>(sh, ni, d.nyg - 2, nk, nmem);
+    const int kc = pk.kc;
+    dim3 blk(pk.tx, pk.ty, 1);
     PROF_BEGIN("k_rhs_rk", s);
 #define RHS_MODE(TX, TY, M)                                                                                         \
     do {                                                                                                            \
@@ -413,14 +465,13 @@ void run_rhs_rk(const RhsArgs<T>& one, const RhsArgs<T>* tab, int nmem, const Di
     } while (0)
 #define RHS_GO(TX, TY)                                                                                              \
     do {                                                                                                            \
-        const int kc = std::min(RHS_KMAX, sh.kchunk > 0 ? sh.kchunk : rhs_round_chunk<T, TX, TY>(ni, d.nyg - 2, nk, nmem)); \
         dim3 grd(cdiv(ni, TX), cdiv(d.nyg - 2, TY), (unsigned)cdiv(nk, kc) * nmem);                                 \
         if (mode == 0) RHS_MODE(TX, TY, 0);                                                                         \
         else if (mode == 1) RHS_MODE(TX, TY, 1);                                                                    \
         else RHS_MODE(TX, TY, 2);                                                                                   \
     } while (0)
-    if (sh.tx == 64 && sh.ty == 4) RHS_GO(64, 4);
-    else if (sh.tx == 64 && sh.ty == 8) RHS_GO(64, 8);
+    if (pk.tx == 64 && pk.ty == 4) RHS_GO(64, 4);
+    else if (pk.tx == 64 && pk.ty == 8) RHS_GO(64, 8);
     else RHS_GO(32, 8);
 #undef RHS_GO
 #undef RHS_MODE
