@@ -512,6 +512,21 @@ int scratch_address(chan_ctx* c)
     return CHAN_OK;
 }
 
+// Transforms per block of an FFT pass over `rows` transforms of length N (any
+// number gives the same bits).  About 384 blocks, so that a small grid uses
+// more of the chip: of the step's time per substep, 128x40x64 FP64 101 us with
+// 4 z-row pairs per block against 109 with 16, 96x64x96 134.8 with 8 against
+// 138.3, 120x58x90 145 with 7 against 150.  At most 8 (128x96x128 213.9 us
+// against 216.6 with 16, 192x96x192 373.3 against 375.1), but 16 for the many
+// rows of a group (the 64-channel ensemble 631 ms per 100 steps against 655);
+// at least 3 (runs of 6 z values on the transposing side); at most the 2048
+// elements a block's registers take.
+int fft_batch(long rows, int N)
+{
+    const int most = rows < 64L * 384 ? 8 : 16;
+    return std::max(1, std::min({2048 / N, most, std::max(3, cdiv(rows, 384))}));
+}
+
 }  // namespace
 
 // ================================================================ C ABI
@@ -725,8 +740,8 @@ int chan_create(const chan_config* cfg, chan_ctx** out)
     c->pb.fx = fx;
     c->pb.fz = fz;
     if ((rc = make_twiddles(c, c->pb.fx)) || (rc = make_twiddles(c, c->pb.fz))) return rc;
-    c->pb.bx = std::max(1, std::min(16, 2048 / d.nxp));
-    c->pb.bz = std::max(1, std::min(16, 2048 / d.nzp));
+    c->pb.bx = fft_batch((long)(d.ny - 1) * (d.nzp / 2), d.nxp);
+    c->pb.bz = fft_batch((long)(d.ny - 1) * d.nkx, d.nzp);
     if (tridiag_needs_table(d)) {
         if ((rc = dalloc(c, (void**)&c->pb.tri, (size_t)(d.ny - 1) * d.nzp * d.nkx * sizeof(double)))) return rc;
         launch_tridiag_setup(d, c->pb, c->stream);
@@ -1685,9 +1700,13 @@ int enqueue_group_step(chan_ensemble* e, const std::vector<int>& idx, TabSink& s
             const PoissonBufs* tp = sink.put(pbv);
             const ProjArgs<T>* tr = sink.put(pr);
             if (sink.launch) {
-                run_poisson_forward<T>(f[0], tf, tp, n, d, c0->pb, s);
-                run_poisson_solve(c0->pb, tp, n, d, s);
-                run_poisson_inverse(c0->pb, tp, n, d, s);
+                // the group's batches: as a channel's, over all members
+                PoissonBufs pb0 = c0->pb;
+                pb0.bx = fft_batch((long)n * (d.ny - 1) * (d.nzp / 2), d.nxp);
+                pb0.bz = fft_batch((long)n * (d.ny - 1) * d.nkx, d.nzp);
+                run_poisson_forward<T>(f[0], tf, tp, n, d, pb0, s);
+                run_poisson_solve(pb0, tp, n, d, s);
+                run_poisson_inverse(pb0, tp, n, d, s);
                 run_project<T>(pr[0], tr, n, d, s);
             }
         }
