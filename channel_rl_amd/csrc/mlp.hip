@@ -72,7 +72,7 @@ struct alignas(16) MlpNet {
 };
 static_assert(sizeof(MlpNet) % 16 == 0, "the image is copied in 16-byte pieces");
 // training also holds the backward operands, A[k = 16m + l%16][n] = W[k][n]
-struct MlpLds : MlpNet {
+struct MlpTrain : MlpNet {
     bf16x8 bw[2][4][2][64];
 };
 
@@ -109,16 +109,16 @@ __device__ void mlp_fill(MlpNet& s, bf16x8 (*bw)[4][2][64], const float* __restr
     if (tid < 2) { s.ym[tid] = norm[8 + tid]; s.ys[tid] = norm[10 + tid]; }
 }
 
-__device__ void mlp_load_lds(MlpLds& s, const float* __restrict__ p, const float* __restrict__ norm)
-{
-    mlp_fill(s, s.bw, p, norm);
-}
-
-// one block: the inference image of the parameters
+// one block: the inference image of the parameters; the training image
 __global__ void __launch_bounds__(256) k_mlp_image(const float* __restrict__ p, const float* __restrict__ norm,
                                                    MlpNet* __restrict__ img)
 {
     mlp_fill(*img, nullptr, p, norm);
+}
+__global__ void __launch_bounds__(256) k_mlp_train_image(const float* __restrict__ p, const float* __restrict__ norm,
+                                                         MlpTrain* __restrict__ img)
+{
+    mlp_fill(*img, img->bw, p, norm);
 }
 
 // the image into a block's LDS
@@ -230,59 +230,132 @@ struct TrainBufs {
     float *Xt, *H[3], *DZ[3], *DY, *loss;
 };
 
-__global__ void __launch_bounds__(256) k_mlp_fwd_bwd(const float* __restrict__ p, const float* __restrict__ norm,
-                                                     const float* __restrict__ X, const float* __restrict__ Tg,
-                                                     const int* __restrict__ idx, int nvalid, int B, TrainBufs tb)
+// One block per 16-sample group, wave m holding the features 16m..16m+15 of
+// every layer (a lane: its sample's features 16m + 4g + r), so the SiLUs and
+// their derivatives, most of the instructions, are spread over four SIMDs;
+// the waves exchange activations through LDS, where the layout above makes a
+// lane's MFMA operand the four waves' 8-byte pieces at its own lane.  The
+// weights come from the training image in global memory, eight 16-byte loads a
+// lane in flight from the start.  The arithmetic and its order are those of
+// mlp_forward.  A batch of 1024: 14.4 us when a wave took whole groups and
+// every block gathered the image from the FP32 parameters into LDS, 7.2 now:
+// two dependent loads (index, sample), five exchanges and the launch itself.
+__global__ void __launch_bounds__(256) k_mlp_fwd_bwd(const MlpTrain* __restrict__ img, const float* __restrict__ X,
+                                                     const float* __restrict__ Tg, const int* __restrict__ idx,
+                                                     int nvalid, int B, TrainBufs tb)
 {
-    __shared__ MlpLds s;
-    mlp_load_lds(s, p, norm);
-    __syncthreads();
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, g = lane / 16;
-    const int ngroups = B / 16;
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    __shared__ bf16x4 ex[4][4][64];  // [exchange][wave][lane]
+    __shared__ floatx4 eh[4][64];
+    const int lane = threadIdx.x % 64, m = threadIdx.x / 64, g = lane / 16;
+    const int grp = blockIdx.x, sl = grp * 16 + lane % 16;  // slot in the batch
+    const int n0 = 16 * m + 4 * g;                          // this lane's features n0 + r
+    const bool ok = sl < nvalid;
     const float inv = 1.0f / (float)nvalid;
-    for (int grp = blockIdx.x * 4 + wave; grp < ngroups; grp += gridDim.x * 4) {
-        lds_reload_fence();
-        const int sl = grp * 16 + lane % 16;  // slot in the batch
-        const bool ok = sl < nvalid;
-        const long src = ok ? (long)idx[sl] : 0;
-        float x[4], t[2];
-        for (int k = 0; k < 4; k++) x[k] = ok ? (X[src * 4 + k] - s.xm[k]) / s.xs[k] : 0.f;
-        for (int m = 0; m < 2; m++) t[m] = ok ? (Tg[src * 2 + m] - s.ym[m]) / s.ys[m] : 0.f;
-        Act z1, z2, z3, h3q;
-        float y[2];
-        mlp_forward(s, x, z1, z2, z3, h3q, y);
-        float dy[2], l2 = 0.f;
-        for (int m = 0; m < 2; m++) {
-            const float e = ok ? y[m] - t[m] : 0.f;
-            dy[m] = e * inv;
-            l2 += e * e;
+    const long src = ok ? (long)idx[sl] : 0;
+    bf16x8 fw[2][2], bw[2][2];
+    for (int L = 0; L < 2; L++)
+        for (int q = 0; q < 2; q++) {
+            fw[L][q] = img->fw[L][m][q][lane];
+            bw[L][q] = img->bw[L][m][q][lane];
         }
-        // backward through the output layer and the SiLUs
-        Act dz3, dz2, dz1, dh;
-        for (int q = 0; q < 16; q++) {
-            const int n = 16 * (q / 4) + 4 * g + (q % 4);
-            dz3.a[q] = (s.w4[n * 2 + 0] * dy[0] + s.w4[n * 2 + 1] * dy[1]) * dsilu(z3.a[q]);
+    floatx4 w1[4], w4[4][2];
+    for (int k = 0; k < 4; k++) w1[k] = *reinterpret_cast<const floatx4*>(&img->w1[k * 64 + n0]);
+    const floatx4 b1 = *reinterpret_cast<const floatx4*>(&img->b1[n0]);
+    const floatx4 b2 = *reinterpret_cast<const floatx4*>(&img->b2[n0]);
+    const floatx4 b3 = *reinterpret_cast<const floatx4*>(&img->b3[n0]);
+    for (int t = 0; t < 4; t++)
+        for (int h = 0; h < 2; h++) w4[t][h] = *reinterpret_cast<const floatx4*>(&img->w4[(16 * t + 4 * g) * 2 + 4 * h]);
+    float x[4], t[2];
+    for (int k = 0; k < 4; k++) x[k] = ok ? (X[src * 4 + k] - img->xm[k]) / img->xs[k] : 0.f;
+    for (int c = 0; c < 2; c++) t[c] = ok ? (Tg[src * 2 + c] - img->ym[c]) / img->ys[c] : 0.f;
+    // the product of one layer for this wave's 16 features, from every wave's v
+    auto layer = [&](int e, const bf16x8 (&A)[2], const float (&v)[4], float (&out)[4]) {
+        bf16x4 h;
+        for (int r = 0; r < 4; r++) h[r] = (__bf16)v[r];
+        ex[e][m][lane] = h;
+        __syncthreads();
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int q = 0; q < 2; q++) {
+            const bf16x4 lo = ex[e][2 * q][lane], hi = ex[e][2 * q + 1][lane];
+            bf16x8 bq;
+            for (int r = 0; r < 4; r++) {
+                bq[r] = lo[r];
+                bq[4 + r] = hi[r];
+            }
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[q], bq, acc, 0, 0, 0);
         }
-        mfma_layer(s.bw[1], dz3, dh, lane);  // dH2 = W3 dZ3
-        for (int q = 0; q < 16; q++) dz2.a[q] = dh.a[q] * dsilu(z2.a[q]);
-        mfma_layer(s.bw[0], dz2, dh, lane);  // dH1 = W2 dZ2
-        for (int q = 0; q < 16; q++) dz1.a[q] = dh.a[q] * dsilu(z1.a[q]);
-        // per-sample quantities, feature-major
-        for (int q = 0; q < 16; q++) {
-            const int n = 16 * (q / 4) + 4 * g + (q % 4);
-            const long o = (long)n * B + sl;
-            tb.H[0][o] = bfr(silu(z1.a[q]));
-            tb.H[1][o] = bfr(silu(z2.a[q]));
-            tb.H[2][o] = h3q.a[q];
-            tb.DZ[0][o] = ok ? dz1.a[q] : 0.f;
-            tb.DZ[1][o] = ok ? dz2.a[q] : 0.f;
-            tb.DZ[2][o] = ok ? dz3.a[q] : 0.f;
+        for (int r = 0; r < 4; r++) out[r] = acc[r];
+    };
+    float z1[4], z2[4], z3[4], h1[4], h2[4], h3q[4];
+    for (int r = 0; r < 4; r++) {
+        float z = b1[r];
+        for (int k = 0; k < 4; k++) z += x[k] * w1[k][r];
+        z1[r] = z;
+        h1[r] = silu(z);
+    }
+    layer(0, fw[0], h1, z2);
+    for (int r = 0; r < 4; r++) {
+        z2[r] += b2[r];
+        h2[r] = silu(z2[r]);
+    }
+    layer(1, fw[1], h2, z3);
+    for (int r = 0; r < 4; r++) {
+        z3[r] += b3[r];
+        h3q[r] = bfr(silu(z3[r]));
+    }
+    eh[m][lane] = floatx4{h3q[0], h3q[1], h3q[2], h3q[3]};
+    __syncthreads();
+    // every wave sums the output layer over all features, in one order
+    float y0 = 0.f, y1 = 0.f;
+    for (int q = 0; q < 16; q++) {
+        const float h = eh[q / 4][lane][q % 4];
+        y0 += h * w4[q / 4][(q % 4) / 2][2 * (q % 2)];
+        y1 += h * w4[q / 4][(q % 4) / 2][2 * (q % 2) + 1];
+    }
+    y0 += __shfl_xor(y0, 16);
+    y1 += __shfl_xor(y1, 16);
+    y0 += __shfl_xor(y0, 32);
+    y1 += __shfl_xor(y1, 32);
+    const float y[2] = {y0 + img->b4[0], y1 + img->b4[1]};
+    float dy[2], l2 = 0.f;
+    for (int c = 0; c < 2; c++) {
+        const float e = ok ? y[c] - t[c] : 0.f;
+        dy[c] = e * inv;
+        l2 += e * e;
+    }
+    // backward through the output layer and the SiLUs
+    float dz3[4], dz2[4], dz1[4], dh[4];
+    for (int r = 0; r < 4; r++) {
+        // w4 of this wave's tile by a uniform selection (a register array
+        // indexed by m would live in scratch memory)
+        float wa = w4[0][r / 2][2 * (r % 2)], wb = w4[0][r / 2][2 * (r % 2) + 1];
+        for (int q = 1; q < 4; q++) {
+            wa = m == q ? w4[q][r / 2][2 * (r % 2)] : wa;
+            wb = m == q ? w4[q][r / 2][2 * (r % 2) + 1] : wb;
         }
-        if (lane < 16) {
-            for (int k = 0; k < 4; k++) tb.Xt[(long)k * B + sl] = x[k];
-            tb.DY[sl] = dy[0];
-            tb.DY[(long)B + sl] = dy[1];
-        }
+        dz3[r] = (wa * dy[0] + wb * dy[1]) * dsilu(z3[r]);
+    }
+    layer(2, bw[1], dz3, dh);  // dH2 = W3 dZ3
+    for (int r = 0; r < 4; r++) dz2[r] = dh[r] * dsilu(z2[r]);
+    layer(3, bw[0], dz2, dh);  // dH1 = W2 dZ2
+    for (int r = 0; r < 4; r++) dz1[r] = dh[r] * dsilu(z1[r]);
+    // per-sample quantities, feature-major
+    for (int r = 0; r < 4; r++) {
+        const long o = (long)(n0 + r) * B + sl;
+        tb.H[0][o] = bfr(h1[r]);
+        tb.H[1][o] = bfr(h2[r]);
+        tb.H[2][o] = h3q[r];
+        tb.DZ[0][o] = ok ? dz1[r] : 0.f;
+        tb.DZ[1][o] = ok ? dz2[r] : 0.f;
+        tb.DZ[2][o] = ok ? dz3[r] : 0.f;
+    }
+    if (m == 0 && lane < 16) {
+        for (int k = 0; k < 4; k++) tb.Xt[(long)k * B + sl] = x[k];
+        tb.DY[sl] = dy[0];
+        tb.DY[(long)B + sl] = dy[1];
+    }
+    if (m == 0) {
         // loss partial of this group: lanes 0..15 hold one sample each
         float lsum = lane < 16 ? l2 : 0.f;
         for (int o = 8; o >= 1; o >>= 1) lsum += __shfl_xor(lsum, o);
@@ -290,83 +363,190 @@ __global__ void __launch_bounds__(256) k_mlp_fwd_bwd(const float* __restrict__ p
     }
 }
 
-// Weight gradients.  Blocks 0..7: one wave per 16x16 tile of dW2 / dW3 =
-// sum_s H_{L-1}[k][s] dZ_L[n][s] on the matrix cores (operands rounded to
-// BF16, K = 32 samples per instruction).  Blocks 8..: one wave per small
-// parameter (W1, b1..b3, W4, b4; 578 of them), its lanes striding over the
-// samples (coalesced rows of the feature-major buffers), then a butterfly
-// over the lanes.  Every sum runs in a fixed order.
-constexpr int MLP_SMALL = 578;
-constexpr int MLP_WGRAD_BLOCKS = 8 + (MLP_SMALL + 3) / 4;
-__global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, int B, float* __restrict__ grad)
+// Adam (Kingma & Ba 2015) on the FP32 master parameters; c1 = 1/(1-b1^t),
+// c2 = 1/(1-b2^t) from the host.  The training image takes the new values.
+struct AdamArgs {
+    float *p, *m, *v;
+    MlpTrain* img;
+    float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ float adam(const AdamArgs& a, int q, float gq, float pq, float m0, float v0)
 {
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, g = lane / 16;
-    if (blockIdx.x < 8) {
-        const int tile = blockIdx.x * 4 + wave;  // 0..31
-        const int L = tile / 16, mk = (tile / 4) % 4, mn = tile % 4;
-        const float* H = tb.H[L];       // H1 for dW2, H2 for dW3
-        const float* DZ = tb.DZ[L + 1]; // dZ2, dZ3
-        const int k = 16 * mk + lane % 16, n = 16 * mn + lane % 16;
-        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int c = 0; c < B / 32; c++) {
-            bf16x8 a, b;
-            const long s0 = (long)c * 32 + 8 * g;
-            for (int e = 0; e < 8; e++) {
-                a[e] = (__bf16)H[(long)k * B + s0 + e];
-                b[e] = (__bf16)DZ[(long)n * B + s0 + e];
-            }
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-        }
-        float* dW = grad + (L == 0 ? MLP_W2 : MLP_W3);
-        for (int r = 0; r < 4; r++) dW[(16 * mk + 4 * g + r) * 64 + n] = acc[r];
-        return;
-    }
-    // small parameters: 256 (W1) + 64 x 3 (biases) + 128 (W4) + 2 (b4)
-    const int q = (blockIdx.x - 8) * 4 + wave;
-    if (q >= MLP_SMALL) return;
-    const float *A = nullptr, *Bv = nullptr;  // the sum of A[s] * Bv[s] (Bv null: of A[s])
-    float* out;
-    if (q < 256) {
-        const int k = q / 64, n = q % 64;
-        A = tb.DZ[0] + (long)n * B;
-        Bv = tb.Xt + (long)k * B;
-        out = grad + MLP_W1 + q;
-    } else if (q < 448) {
-        const int L = (q - 256) / 64, n = (q - 256) % 64;
-        A = tb.DZ[L] + (long)n * B;
-        out = grad + (L == 0 ? MLP_B1 : (L == 1 ? MLP_B2 : MLP_B3)) + n;
-    } else if (q < 576) {
-        const int n = (q - 448) / 2, m = (q - 448) % 2;
-        A = tb.H[2] + (long)n * B;
-        Bv = tb.DY + (long)m * B;
-        out = grad + MLP_W4 + q - 448;
-    } else {
-        A = tb.DY + (long)(q - 576) * B;
-        out = grad + MLP_B4 + q - 576;
-    }
-    float sum = 0.f;
-    if (Bv) {
-        for (int s = lane; s < B; s += 64) sum += A[s] * Bv[s];
-    } else {
-        for (int s = lane; s < B; s += 64) sum += A[s];
-    }
-    for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
-    if (lane == 0) *out = sum;
+    const float mq = a.b1 * m0 + (1.0f - a.b1) * gq;
+    const float vq = a.b2 * v0 + (1.0f - a.b2) * gq * gq;
+    const float pn = pq - a.lr * (mq * a.c1) / (sqrtf(vq * a.c2) + a.eps);
+    a.m[q] = mq;
+    a.v[q] = vq;
+    a.p[q] = pn;
+    return pn;
+}
+// the element of an MFMA operand image [m][q][lane][e] (perm_feature) that
+// holds row (the m, lane%16 side) and reduction index k
+__device__ __forceinline__ int image_at(int row, int k)
+{
+    const int kt = k / 16, e = 4 * (kt % 2) + k % 4, lane = 16 * ((k % 16) / 4) + row % 16;
+    return (((row / 16) * 2 + kt / 2) * 64 + lane) * 8 + e;
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master parameters; c1 = 1/(1-b1^t),
-// c2 = 1/(1-b2^t) from the host.
-__global__ void k_mlp_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                           const float* __restrict__ grad, float lr, float b1, float b2, float eps, float c1, float c2)
+// Weight gradients and, with ADAM, the optimiser step on them (without: the
+// gradients to grad).  Every sum runs in a fixed order.
+// Blocks 0..31: one 16x16 tile of dW2 / dW3 = sum_s H_{L-1}[k][s] dZ_L[n][s]
+// on the matrix cores (operands rounded to BF16, K = 32 samples per
+// instruction).  Four waves bring the operands of up to 1024 samples into LDS,
+// all loads in flight at once, then one wave runs the chain of products.
+// Blocks 32..: the small parameters, one wave per feature row of the
+// sample-major buffers (dW1 and db1 of a feature from one pass over its row,
+// db2, db3, dW4, db4), lanes striding over the samples, then a butterfly.
+// A batch of 1024: 15.7 us when each wave fetched its operands step by step,
+// plus 4.1 for the optimiser in a launch of its own; 6.9 for both now, of which
+// the launch is 4.5.
+constexpr int MLP_WCHUNK = 32;  // products (of 32 samples) per LDS fill
+constexpr int MLP_ROWS = 64 + 128 + 64 + 1;
+constexpr int MLP_WGRAD_BLOCKS = 32 + (MLP_ROWS + 3) / 4;
+template <bool ADAM>
+__global__ void __launch_bounds__(256) k_mlp_wgrad(TrainBufs tb, int B, float* __restrict__ grad, AdamArgs ad)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= MLP_NPARAM) return;
-    const float gq = grad[q];
-    const float mq = b1 * m[q] + (1.0f - b1) * gq;
-    const float vq = b2 * v[q] + (1.0f - b2) * gq * gq;
-    m[q] = mq;
-    v[q] = vq;
-    p[q] = p[q] - lr * (mq * c1) / (sqrtf(vq * c2) + eps);
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64, g = lane / 16;
+    if (blockIdx.x < 32) {
+        __shared__ bf16x8 sa[MLP_WCHUNK][64], sb[MLP_WCHUNK][64];
+        __shared__ float res[16][16];
+        const int tile = blockIdx.x;
+        const int L = tile / 16, mk = (tile / 4) % 4, mn = tile % 4;
+        // the tile's parameter of this thread: W[k][n]
+        const int pk = 16 * mk + threadIdx.x / 16, pn = 16 * mn + threadIdx.x % 16;
+        const int pq = (L == 0 ? MLP_W2 : MLP_W3) + pk * 64 + pn;
+        float p0 = 0.f, m0 = 0.f, v0 = 0.f;
+        if (ADAM) { p0 = ad.p[pq]; m0 = ad.m[pq]; v0 = ad.v[pq]; }
+        const float* H = tb.H[L] + (long)(16 * mk + lane % 16) * B + 8 * g;         // H1 for dW2, H2 for dW3
+        const float* DZ = tb.DZ[L + 1] + (long)(16 * mn + lane % 16) * B + 8 * g;   // dZ2, dZ3
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        const int nc = B / 32;
+        for (int c0 = 0; c0 < nc; c0 += MLP_WCHUNK) {
+            const int cn = min(MLP_WCHUNK, nc - c0);
+            constexpr int U = MLP_WCHUNK / 4;
+            floatx4 ha[U][2], da[U][2];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                // steps past the last re-read it and are not stored
+                const long o = (long)(c0 + min(wave + 4 * u, cn - 1)) * 32;
+                for (int h = 0; h < 2; h++) {
+                    ha[u][h] = *reinterpret_cast<const floatx4*>(H + o + 4 * h);
+                    da[u][h] = *reinterpret_cast<const floatx4*>(DZ + o + 4 * h);
+                }
+            }
+            if (c0) __syncthreads();
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int c = wave + 4 * u;
+                bf16x8 a, b;
+                for (int e = 0; e < 8; e++) {
+                    a[e] = (__bf16)ha[u][e / 4][e % 4];
+                    b[e] = (__bf16)da[u][e / 4][e % 4];
+                }
+                if (c < cn) {
+                    sa[c][lane] = a;
+                    sb[c][lane] = b;
+                }
+            }
+            __syncthreads();
+            if (wave == 0) {
+                int c = 0;
+                for (; c + 8 <= cn; c += 8)
+#pragma unroll
+                    for (int u = 0; u < 8; u++)
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sa[c + u][lane], sb[c + u][lane], acc, 0, 0, 0);
+                for (; c < cn; c++)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sa[c][lane], sb[c][lane], acc, 0, 0, 0);
+            }
+        }
+        if (wave == 0)
+            for (int r = 0; r < 4; r++) res[4 * g + r][lane % 16] = acc[r];
+        __syncthreads();
+        const float gq = res[threadIdx.x / 16][threadIdx.x % 16];
+        if (ADAM) {
+            const __bf16 w = (__bf16)adam(ad, pq, gq, p0, m0, v0);
+            reinterpret_cast<__bf16*>(ad.img->fw[L])[image_at(pn, pk)] = w;  // A[n][k]
+            reinterpret_cast<__bf16*>(ad.img->bw[L])[image_at(pk, pn)] = w;  // A[k][n]
+        } else {
+            grad[pq] = gq;
+        }
+        return;
+    }
+    const int q = (blockIdx.x - 32) * 4 + wave;
+    if (q >= MLP_ROWS) return;
+    // up to five sums of one row: A[s] * Bv[j][s], and A[s]
+    const float *A, *Bv = nullptr;
+    int out[5] = {0, 0, 0, 0, 0}, np;
+    if (q < 64) {  // W1[k][q], b1[q]
+        A = tb.DZ[0] + (long)q * B;
+        Bv = tb.Xt;
+        for (int k = 0; k < 4; k++) out[k] = MLP_W1 + k * 64 + q;
+        out[4] = MLP_B1 + q;
+        np = 5;
+    } else if (q < 192) {  // b2, b3
+        A = tb.DZ[1 + (q - 64) / 64] + (long)(q % 64) * B;
+        out[4] = (q < 128 ? MLP_B2 : MLP_B3) + q % 64;
+        np = 5;
+    } else if (q < 256) {  // W4[n][.]
+        A = tb.H[2] + (long)(q - 192) * B;
+        Bv = tb.DY;
+        out[0] = MLP_W4 + 2 * (q - 192);
+        out[1] = out[0] + 1;
+        np = 2;
+    } else {  // b4
+        A = tb.DY;
+        out[0] = MLP_B4;
+        out[1] = MLP_B4 + 1;
+        np = 2;
+    }
+    float sum[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    // B is a multiple of 32: whole turns of the wave, then half a turn
+    auto sweep = [&](auto&& add) {
+#pragma unroll 8
+        for (int t = 0; t < B / 64; t++) add(64 * t + lane);
+        if (B % 64 && lane < 32) add(B - 32 + lane);
+    };
+    if (q < 64) {
+        sweep([&](int s) {
+            const float a = A[s];
+            for (int k = 0; k < 4; k++) sum[k] += a * Bv[(long)k * B + s];
+            sum[4] += a;
+        });
+    } else if (q < 192) {
+        sweep([&](int s) { sum[4] += A[s]; });
+    } else if (q < 256) {
+        sweep([&](int s) {
+            const float a = A[s];
+            sum[0] += a * Bv[s];
+            sum[1] += a * Bv[(long)B + s];
+        });
+    } else {
+        sweep([&](int s) {
+            sum[0] += A[s];
+            sum[1] += A[(long)B + s];
+        });
+    }
+    for (int k = 0; k < 5; k++)
+        for (int o = 32; o >= 1; o >>= 1) sum[k] += __shfl_xor(sum[k], o);
+    // lane k takes sum k
+    float gq = sum[0];
+    int pq = out[0];
+    for (int k = 1; k < 5; k++)
+        if (lane == k) { gq = sum[k]; pq = out[k]; }
+    const bool mine = lane < np && !(q >= 64 && q < 192 && lane != 4);
+    if (!mine) return;
+    if (!ADAM) {
+        grad[pq] = gq;
+        return;
+    }
+    const float pn = adam(ad, pq, gq, ad.p[pq], ad.m[pq], ad.v[pq]);
+    MlpTrain& im = *ad.img;
+    if (q < 64) {
+        if (lane < 4) im.w1[pq - MLP_W1] = bfr(pn);
+        else im.b1[q] = pn;
+    } else if (q < 192) (q < 128 ? im.b2 : im.b3)[q % 64] = pn;
+    else if (q < 256) im.w4[pq - MLP_W4] = bfr(pn);
+    else im.b4[lane] = pn;
 }
 
 // --------------------------------------------------------- the wall model
@@ -586,6 +766,7 @@ struct chan_mlp {
     hipStream_t stream = nullptr;
     float *p = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr, *norm = nullptr;
     MlpNet* img = nullptr;
+    MlpTrain* timg = nullptr;  // the training kernels' image, filled when a training call begins
     hipEvent_t ready = nullptr;
     std::mutex mu;
     struct User {
@@ -719,16 +900,13 @@ int end_update(chan_mlp* c)
 // one optimiser step on the batch idx[0..nvalid) (already on the device)
 int train_batch(chan_mlp* c, int nvalid, int B, float lr)
 {
-    const int groups = B / 16;
-    const int blocks = std::max(1, (groups + 3) / 4);
-    k_mlp_fwd_bwd<<<blocks, 256, 0, c->stream>>>(c->p, c->norm, c->X, c->Y, c->idx, nvalid, B, c->tb);
-    k_mlp_wgrad<<<MLP_WGRAD_BLOCKS, 256, 0, c->stream>>>(c->tb, B, c->grad);
+    k_mlp_fwd_bwd<<<B / 16, 256, 0, c->stream>>>(c->timg, c->X, c->Y, c->idx, nvalid, B, c->tb);
     c->adam_t++;
     const double b1 = 0.9, b2 = 0.999;
     const float c1 = (float)(1.0 / (1.0 - std::pow(b1, c->adam_t)));
     const float c2 = (float)(1.0 / (1.0 - std::pow(b2, c->adam_t)));
-    k_mlp_adam<<<cdiv(MLP_NPARAM, 256), 256, 0, c->stream>>>(c->p, c->m, c->v, c->grad, lr, (float)b1, (float)b2,
-                                                             1e-8f, c1, c2);
+    const AdamArgs ad{c->p, c->m, c->v, c->timg, lr, (float)b1, (float)b2, 1e-8f, c1, c2};
+    k_mlp_wgrad<true><<<MLP_WGRAD_BLOCKS, 256, 0, c->stream>>>(c->tb, B, nullptr, ad);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return mfail(c, CHAN_EHIP, std::string("mlp training launch: ") + hipGetErrorString(e));
     return CHAN_OK;
@@ -753,6 +931,7 @@ int chan_mlp_create(int device, unsigned long long seed, chan_mlp** out)
     MCHK(c, hipMalloc(&c->grad, MLP_NPARAM * sizeof(float)));
     MCHK(c, hipMalloc(&c->norm, MLP_NNORM * sizeof(float)));
     MCHK(c, hipMalloc(&c->img, sizeof(MlpNet)));
+    MCHK(c, hipMalloc(&c->timg, sizeof(MlpTrain)));
     MCHK(c, hipEventCreateWithFlags(&c->ready, hipEventDisableTiming));
     // He-uniform weights (bound sqrt(6 / fan_in)), zero biases, identity
     // standardisation; seeded counter RNG
@@ -793,6 +972,7 @@ int chan_mlp_destroy(chan_mlp* c)
     for (float* b : bufs)
         if (b) (void)hipFree(b);
     if (c->img) (void)hipFree(c->img);
+    if (c->timg) (void)hipFree(c->timg);
     if (c->idx) (void)hipFree(c->idx);
     if (c->ready) (void)hipEventDestroy(c->ready);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -866,9 +1046,9 @@ int chan_mlp_gradients(chan_mlp* c, const float* X, const float* Y, int n, float
     MCHK(c, hipMemcpyAsync(c->Y, Y, (size_t)n * 2 * sizeof(float), hipMemcpyHostToDevice, c->stream));
     MCHK(c, hipMemcpyAsync(c->idx, id.data(), (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->stream));
     const int groups = B / 16;
-    k_mlp_fwd_bwd<<<std::max(1, (groups + 3) / 4), 256, 0, c->stream>>>(c->p, c->norm, c->X, c->Y, c->idx, n, B,
-                                                                        c->tb);
-    k_mlp_wgrad<<<MLP_WGRAD_BLOCKS, 256, 0, c->stream>>>(c->tb, B, c->grad);
+    k_mlp_train_image<<<1, 256, 0, c->stream>>>(c->p, c->norm, c->timg);
+    k_mlp_fwd_bwd<<<groups, 256, 0, c->stream>>>(c->timg, c->X, c->Y, c->idx, n, B, c->tb);
+    k_mlp_wgrad<false><<<MLP_WGRAD_BLOCKS, 256, 0, c->stream>>>(c->tb, B, c->grad, AdamArgs{});
     MCHK(c, hipGetLastError());
     std::vector<float> lp(groups);
     MCHK(c, hipMemcpyAsync(grad, c->grad, MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, c->stream));
@@ -928,6 +1108,7 @@ int chan_mlp_train(chan_mlp* c, const float* X, const float* Y, int n, int epoch
         (void)hipFree(dperm);
         return mfail(c, CHAN_ENOMEM, "mlp train: loss buffer");
     }
+    k_mlp_train_image<<<1, 256, 0, c->stream>>>(c->p, c->norm, c->timg);
     uint64_t st = seed;
     std::vector<float> lp((size_t)nb * (batch / 16));
     float* keep_loss = c->tb.loss;
