@@ -908,39 +908,95 @@ void launch_poisson_inverse(const Dims& d, PoissonBufs& pb, hipStream_t s)
 // code/projection.f90:192-214: u -= grad p on the canonical cells, each
 // stored with its boundary-condition images (the reference applies
 // apply_boundary_conditions right after, code/time_integration.f90:49).
-template <typename T, bool G>
+// HBM-bound.  A lane takes KZ cells along z and issues all of their loads
+// before the first store, so that a wave keeps enough in flight (one FP32 cell
+// a lane moves 32 bytes); p(k+1) of one cell is p(k) of the next, and the x and
+// y factors are read once.  Only the cells of the box's faces, edges and
+// corners have images and go through store_img.
+template <typename T, int KZ, bool G>
 __global__ void __launch_bounds__(256) k_project(ProjArgs<T> one, const ProjArgs<T>* tab, Dims d)
 {
     // XCD-contiguous tile order: the plane k+1 that a tile reads is the
     // plane k of a tile that runs on the same XCD, so p is fetched once
-    const GBlk gb = gblk_xcd(d.nzg - 3);
+    const int nz = d.nzg - 3;
+    const GBlk gb = gblk_xcd((nz + KZ - 1) / KZ);
     const ProjArgs<T> arg = member_args<G>(one, tab, gb.m);
-    T *U = arg.U, *V = arg.V, *W = arg.W;
     const double* __restrict__ p = arg.p;
     const Metric<double>& m = arg.m;
-    const TileId t{gb.x, gb.y, gb.z};
-    const int i = t.x * blockDim.x + threadIdx.x + 2;
-    const int j = t.y * blockDim.y + threadIdx.y + 2;
-    const int k = t.z + 2;
+    const int i = gb.x * blockDim.x + threadIdx.x + 2;
+    const int j = gb.y * blockDim.y + threadIdx.y + 2;
+    const int k0 = gb.z * KZ + 2;
     if (i > d.nxg - 2 || j > d.nyg - 1) return;
-    const long q = at(d, i, j, k);
-    const double p0 = p[q];
-    // the spacings' reciprocals: within an ulp of the reference's divisions
-    const T un = T((double)U[q] - (p[at(d, i + 1, j, k)] - p0) * m.rdxg[i + 1]);
-    store_img(U, d, 0, i, j, k, arg.shift ? un + T(arg.shift->last_dPdx) : un);
-    if (j <= d.ny - 1)
-        store_img(V, d, 1, i, j, k, T((double)V[q] - (p[at(d, i, j + 1, k)] - p0) * m.rdyg[j + 1]));
-    store_img(W, d, 2, i, j, k, T((double)W[q] - (p[at(d, i, j, k + 1)] - p0) * m.rdzg[k + 1]));
+    const int last = min(KZ, nz + 2 - k0) - 1;  // the lane's last cell
+    const long q = at(d, i, j, k0);
+    T* __restrict__ const U = arg.U;
+    T* __restrict__ const V = arg.V;
+    T* __restrict__ const W = arg.W;
+    const double rx = m.rdxg[i + 1], ry = m.rdyg[min(j + 1, d.nyg)];
+    T u[KZ], v[KZ], w[KZ];
+    double pc[KZ + 1], px[KZ], py[KZ];
+    pc[0] = p[q];
+#pragma unroll
+    for (int t = 0; t < KZ; t++) {
+        // cells past the last plane read the last one again
+        const long c = q + (long)min(t, last) * d.sxy;
+        u[t] = U[c];
+        v[t] = V[c];
+        w[t] = W[c];
+        px[t] = p[c + 1];
+        py[t] = p[c + d.sx];
+        pc[t + 1] = p[c + d.sxy];
+    }
+    const T shift = arg.shift ? T(arg.shift->last_dPdx) : T(0);
+    const bool vrow = j <= d.ny - 1;
+    const bool face = i <= 3 || i >= d.nxg - 2 || j == 2 || j == d.nyg - 1;
+#pragma unroll
+    for (int t = 0; t < KZ; t++) {
+        if (t > last) break;
+        const int k = k0 + t;
+        const long c = q + (long)t * d.sxy;
+        // the spacings' reciprocals: within an ulp of the reference's divisions
+        const double p0 = pc[t];
+        T un = T((double)u[t] - (px[t] - p0) * rx);
+        if (arg.shift) un = un + shift;
+        const T vn = T((double)v[t] - (py[t] - p0) * ry);
+        const T wn = T((double)w[t] - (pc[t + 1] - p0) * m.rdzg[k + 1]);
+        U[c] = un;
+        if (vrow) V[c] = vn;
+        W[c] = wn;
+        if (face || k <= 3 || k >= d.nzg - 2) {
+            store_img(U, d, 0, i, j, k, un);
+            if (vrow) store_img(V, d, 1, i, j, k, vn);
+            store_img(W, d, 2, i, j, k, wn);
+        }
+    }
+}
+
+template <typename T, int KZ>
+static void go_project(const ProjArgs<T>& one, const ProjArgs<T>* tab, int nmem, const Dims& d, dim3 blk, hipStream_t s)
+{
+    const dim3 grd(cdiv(d.nxg - 3, blk.x), cdiv(d.nyg - 2, blk.y), (unsigned)cdiv(d.nzg - 3, KZ) * nmem);
+    if (tab) k_project<T, KZ, true><<<grd, blk, 0, s>>>(one, tab, d);
+    else k_project<T, KZ, false><<<grd, blk, 0, s>>>(one, nullptr, d);
 }
 
 template <typename T>
 void run_project(const ProjArgs<T>& one, const ProjArgs<T>* tab, int nmem, const Dims& d, hipStream_t s)
 {
     const dim3 blk = row_block(d.nxg - 3);
-    const dim3 grd(cdiv(d.nxg - 3, blk.x), cdiv(d.nyg - 2, blk.y), (unsigned)(d.nzg - 3) * nmem);
+    const long blocks = (long)cdiv(d.nxg - 3, blk.x) * cdiv(d.nyg - 2, blk.y) * (d.nzg - 3) * nmem;
     PROF_BEGIN("k_project", s);
-    if (tab) k_project<T, true><<<grd, blk, 0, s>>>(one, tab, d);
-    else k_project<T, false><<<grd, blk, 0, s>>>(one, nullptr, d);
+    // FP32: four cells a lane once that leaves the chip about 1024 blocks.  In
+    // us, one cell / four: 96x64x96 10.4 / 12.1, 120x58x90 11.5 / 11.4,
+    // 128x96x128 18.6 / 16.2, 192x96x192 32.4 / 25.8 (3.4 -> 4.4 TB/s),
+    // 384x192x384 224 / 221.  FP64 moves enough a cell: 37.2 / 42.1 and
+    // 336 / 355 on the last two.
+    if constexpr (sizeof(T) == 4) {
+        if (blocks >= 4096) go_project<T, 4>(one, tab, nmem, d, blk, s);
+        else go_project<T, 1>(one, tab, nmem, d, blk, s);
+    } else {
+        go_project<T, 1>(one, tab, nmem, d, blk, s);
+    }
     PROF_END(s);
 }
 
