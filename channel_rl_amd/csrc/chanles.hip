@@ -14,6 +14,7 @@
 #include "../../include/chanles.h"
 #include "kernels.hpp"
 #include "prof.hpp"
+#include "readback.hpp"
 #include "wallmodel.hpp"
 
 using namespace chan;
@@ -679,6 +680,7 @@ int chan_create(const chan_config* cfg, chan_ctx** out)
     int rc = set_device(c);
     if (rc) return rc;
     HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    Readback::get().add_channel();
     if ((rc = scratch_address(c))) return rc;
 
     // metrics
@@ -791,7 +793,10 @@ void chan_destroy(chan_ctx* c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->net) mlp_detach(c->net, c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
-    if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (c->stream) {
+        (void)hipStreamDestroy(c->stream);
+        Readback::get().remove_channel();
+    }
     delete c;
 }
 
@@ -838,8 +843,7 @@ int chan_get_field(chan_ctx* c, int which, double* dst)
     else
         k_pack<float><<<cdiv(n, 256), 256, 0, c->stream>>>((const float*)src, c->stage, c->d, s.n1, s.n2, s.n3, s.o);
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipMemcpyAsync(dst, c->stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, Readback::get().copy(dst, c->stage, n * sizeof(double), c->device, c->stream));
     return CHAN_OK;
 }
 
