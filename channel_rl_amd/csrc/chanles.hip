@@ -117,9 +117,10 @@ struct chan_ctx {
     Scalars* sc = nullptr;
     double* mins3 = nullptr;
     PoissonBufs pb{};
-    hipGraphExec_t graph[3] = {nullptr, nullptr, nullptr};
+    // a captured step per rotation of the states, [1]: as a call's last (keep_nut)
+    hipGraphExec_t graph[2][3] = {};
     // the same steps with compute_dt folded into substep 1 (dt_fused)
-    hipGraphExec_t graph_dt[3] = {nullptr, nullptr, nullptr};
+    hipGraphExec_t graph_dt[2][3] = {};
     double* dtpart = nullptr;  // the DSM pass's compute_dt maxima, [3][blocks]
     // substeps 1 and 2 of a step leave the dynamic model's pass B to the RHS
     // kernel (DsmBufs::ntab): its row coefficients, [2][nyg] of the bulk type
@@ -378,8 +379,12 @@ void enqueue_projection(chan_ctx* c, int buf, bool with_mass_flow = false)
 // X (start of step, also Uo), Y, Z; substeps X->Y, Y->Z, Z->Y.
 // dt_fused: compute_dt of the step's start state is taken by the DSM pass
 // of substep 1 and its ratio kernel (dt_fusable), which need it first
+// keep_nut: the call ends with this step, so that the nu_t of its last substep
+// is a field the caller can read.  A step that another follows needs it in the
+// RHS only and defers pass B there too: it saves k_dsm_nut's pass over the box
+// (192x96x192 FP64 17.5 us against 5 of k_dsm_edges, 384x192x384 FP32 57 against 6).
 template <typename T>
-void enqueue_rk3(chan_ctx* c, int X, bool dt_fused = false)
+void enqueue_rk3(chan_ctx* c, int X, bool dt_fused = false, bool keep_nut = true)
 {
     const int Y = (X + 1) % 3, Z = (X + 2) % 3;
     const int in[3] = {X, Y, Z}, out[3] = {Y, Z, Y};
@@ -399,8 +404,8 @@ void enqueue_rk3(chan_ctx* c, int X, bool dt_fused = false)
                 launch_wm_mlp<T>(net, I[0], I[2], c->alpha, c->sc, c->md, c->d, c->nu, c->h_wm, c->kappa, c->Bc,
                                  c->x_mass_cte, c->wm_max_err, c->wm_stats, c->stream);
         }
-        // nu_t is read by the RHS only, except after the last substep
-        const bool defer = c->defer_nut && c->LES_model == 2 && s < 2;
+        // nu_t is read by the RHS only, except after the call's last substep
+        const bool defer = c->defer_nut && c->LES_model == 2 && (s < 2 || !keep_nut);
         enqueue_eddy_viscosity<T>(c, in[s], 1, dt_fused && s == 0, eq_in_dsm, defer);
         double c1, c2 = 0.0;
         if (s == 0) c1 = c->rk_coef[0][0];
@@ -421,13 +426,17 @@ void enqueue_rk3(chan_ctx* c, int X, bool dt_fused = false)
     }
 }
 
+void destroy_graphs(chan_ctx* c)
+{
+    for (auto* of : {&c->graph, &c->graph_dt})
+        for (auto& phase : *of)
+            for (hipGraphExec_t& g : phase)
+                if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
+}
 // the captured steps bake in launch shapes and options: drop them on change
 void drop_graphs(chan_ctx* c)
 {
-    for (int q = 0; q < 3; q++) {
-        if (c->graph[q]) { (void)hipGraphExecDestroy(c->graph[q]); c->graph[q] = nullptr; }
-        if (c->graph_dt[q]) { (void)hipGraphExecDestroy(c->graph_dt[q]); c->graph_dt[q] = nullptr; }
-    }
+    destroy_graphs(c);
     c->generation++;
 }
 
@@ -439,19 +448,21 @@ int check_launch(chan_ctx* c)
 }
 
 template <typename T>
-int rk3_step(chan_ctx* c, bool dt_fused)
+int rk3_step(chan_ctx* c, bool dt_fused, bool keep_nut)
 {
     const int X = c->cur;
+    // one form only where nothing is deferred
+    if (!c->defer_nut || c->LES_model != 2) keep_nut = true;
     if (!c->use_graph) {
-        enqueue_rk3<T>(c, X, dt_fused);
+        enqueue_rk3<T>(c, X, dt_fused, keep_nut);
         int rc = check_launch(c);
         if (rc) return rc;
     } else {
-        hipGraphExec_t& gx = dt_fused ? c->graph_dt[X] : c->graph[X];
+        hipGraphExec_t& gx = (dt_fused ? c->graph_dt : c->graph)[keep_nut][X];
         if (!gx) {
             hipGraph_t g;
             HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            enqueue_rk3<T>(c, X, dt_fused);
+            enqueue_rk3<T>(c, X, dt_fused, keep_nut);
             HIPCHK(c, hipStreamEndCapture(c->stream, &g));
             hipError_t e = hipGraphInstantiate(&gx, g, nullptr, nullptr, 0);
             (void)hipGraphDestroy(g);
@@ -786,10 +797,7 @@ void chan_destroy(chan_ctx* c)
         return;
     }
     (void)hipSetDevice(c->device);
-    for (int q = 0; q < 3; q++) {
-        if (c->graph[q]) (void)hipGraphExecDestroy(c->graph[q]);
-        if (c->graph_dt[q]) (void)hipGraphExecDestroy(c->graph_dt[q]);
-    }
+    destroy_graphs(c);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->net) mlp_detach(c->net, c->stream);
     for (void* p : c->allocs) (void)hipFree(p);
@@ -1058,7 +1066,7 @@ int chan_compute_time_step_RK3(chan_ctx* c)
     int rc = set_device(c);
     if (rc) return rc;
     if ((rc = net_order(c))) return rc;
-    return DISPATCH(c, rk3_step, c, false);
+    return DISPATCH(c, rk3_step, c, false, true);
 }
 
 int chan_check_divergence(chan_ctx* c, double* max_div, double* max_abs)
@@ -1224,12 +1232,12 @@ int chan_run_steps(chan_ctx* c, int nsteps)
             // compute_dt + compute_time_step_RK3 with the former inside the
             // step (the same dt: its maxima are exact in any order)
             if ((rc = net_order(c))) return rc;
-            if ((rc = DISPATCH(c, rk3_step, c, true))) return rc;
+            if ((rc = DISPATCH(c, rk3_step, c, true, n + 1 == nsteps))) return rc;
             continue;
         }
         DISPATCH(c, enqueue_dt, c);
-        if ((rc = check_launch(c))) return rc;
-        if ((rc = chan_compute_time_step_RK3(c))) return rc;
+        if ((rc = check_launch(c)) || (rc = net_order(c))) return rc;
+        if ((rc = DISPATCH(c, rk3_step, c, false, n + 1 == nsteps))) return rc;
     }
     return CHAN_OK;
 }
@@ -1248,7 +1256,7 @@ int chan_profile_steps(chan_ctx* c, int nsteps)
     for (int n = 0; n < nsteps && rc == CHAN_OK; n++) {
         if (fuse) {
             rc = net_order(c);
-            if (!rc) rc = DISPATCH(c, rk3_step, c, true);
+            if (!rc) rc = DISPATCH(c, rk3_step, c, true, true);
         } else {
             DISPATCH(c, enqueue_dt, c);
             rc = check_launch(c);
