@@ -1552,8 +1552,9 @@ struct chan_ensemble {
     hipStream_t stream = nullptr;
     hipEvent_t fork = nullptr, done = nullptr;
     std::vector<hipEvent_t> join;
-    hipGraphExec_t graph[3] = {nullptr, nullptr, nullptr};
-    void* tabmem[3] = {nullptr, nullptr, nullptr};  // argument tables of each graph
+    // a captured step per rotation of the states, 3..5: as a call's last (enqueue_rk3's keep_nut)
+    hipGraphExec_t graph[6] = {};
+    void* tabmem[6] = {};  // argument tables of each graph
     std::vector<int> cur0;    // members' rotation when the graphs were captured
     std::vector<long> gen0;   // members' generation then
     long step = 0;            // steps since the capture base
@@ -1569,7 +1570,7 @@ static int efail(chan_ensemble* e, int code, const std::string& msg)
 
 static void ens_drop(chan_ensemble* e)
 {
-    for (int q = 0; q < 3; q++) {
+    for (int q = 0; q < 6; q++) {
         if (e->graph[q]) { (void)hipGraphExecDestroy(e->graph[q]); e->graph[q] = nullptr; }
         if (e->tabmem[q]) { (void)hipFree(e->tabmem[q]); e->tabmem[q] = nullptr; }
     }
@@ -1619,7 +1620,7 @@ __global__ void k_advance_time_g(const MassArgs<T>* tab) { tab[blockIdx.x].sc->t
 // compute_dt + compute_time_step_RK3 of every member of a group, one launch
 // per stage (the arithmetic of enqueue_dt + enqueue_rk3 per member)
 template <typename T>
-int enqueue_group_step(chan_ensemble* e, const std::vector<int>& idx, TabSink& sink, hipStream_t s)
+int enqueue_group_step(chan_ensemble* e, const std::vector<int>& idx, TabSink& sink, bool keep_nut, hipStream_t s)
 {
     const int n = (int)idx.size();
     chan_ctx* c0 = e->ch[idx[0]];
@@ -1668,8 +1669,8 @@ int enqueue_group_step(chan_ensemble* e, const std::vector<int>& idx, TabSink& s
             if (sink.launch) run_wm_mlp<T>(a[0], t, n, d, s);
         }
         // dynamic Smagorinsky (pass A, plane ratios, pass B with the wall rows;
-        // pass B left to the RHS in substeps 1 and 2, as enqueue_rk3 does)
-        const bool defer = c0->defer_nut && sub < 2;
+        // pass B left to the RHS as enqueue_rk3 does)
+        const bool defer = c0->defer_nut && (sub < 2 || !keep_nut);
         {
             std::vector<DsmArgs<T>> a(n);
             std::vector<DsmRatioArgs> r(n);
@@ -1757,7 +1758,7 @@ int enqueue_group_step(chan_ensemble* e, const std::vector<int>& idx, TabSink& s
 }
 
 // one ensemble step of every group and lone member (sink: see TabSink)
-int enqueue_ensemble_step(chan_ensemble* e, TabSink& sink, hipError_t& h)
+int enqueue_ensemble_step(chan_ensemble* e, TabSink& sink, bool keep_nut, hipError_t& h)
 {
     for (const std::vector<int>& g : e->groups) {
         chan_ctx* c0 = e->ch[g[0]];
@@ -1766,12 +1767,12 @@ int enqueue_ensemble_step(chan_ensemble* e, TabSink& sink, hipError_t& h)
             if (h != hipSuccess) return CHAN_EHIP;
         }
         if (g.size() > 1) {
-            const int rc = c0->prec == CHAN_FP64 ? enqueue_group_step<double>(e, g, sink, c0->stream)
-                                                 : enqueue_group_step<float>(e, g, sink, c0->stream);
+            const int rc = c0->prec == CHAN_FP64 ? enqueue_group_step<double>(e, g, sink, keep_nut, c0->stream)
+                                                 : enqueue_group_step<float>(e, g, sink, keep_nut, c0->stream);
             if (rc) return rc;
         } else if (sink.launch) {
             DISPATCH(c0, enqueue_dt, c0);
-            DISPATCH(c0, enqueue_rk3, c0, c0->cur);
+            DISPATCH(c0, enqueue_rk3, c0, c0->cur, false, keep_nut);
         }
         if (sink.launch) {
             h = hipEventRecord(e->join[g[0]], c0->stream);
@@ -1899,11 +1900,12 @@ int chan_ensemble_run_steps(chan_ensemble* e, int nsteps)
         if (h != hipSuccess) return efail(e, CHAN_EHIP, std::string("ensemble order: ") + hipGetErrorString(h));
     }
     for (int it = 0; it < nsteps; it++) {
-        const int o = (int)(e->step % 3);
+        const bool keep_nut = it + 1 == nsteps;
+        const int o = (int)(e->step % 3) + (keep_nut ? 3 : 0);
         if (!e->graph[o]) {
             // pass 1: the argument tables of this phase, into device memory
             TabSink sink;
-            int rc = enqueue_ensemble_step(e, sink, h);
+            int rc = enqueue_ensemble_step(e, sink, keep_nut, h);
             if (rc) { ens_drop(e); return rc == CHAN_EHIP ? efail(e, rc, hipGetErrorString(h)) : rc; }
             if (!sink.host.empty()) {
                 h = hipMalloc(&e->tabmem[o], sink.host.size());
@@ -1921,7 +1923,7 @@ int chan_ensemble_run_steps(chan_ensemble* e, int nsteps)
             h = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal);
             if (h == hipSuccess) h = hipEventRecord(e->fork, e->stream);
             if (h == hipSuccess) {
-                rc = enqueue_ensemble_step(e, sink, h);
+                rc = enqueue_ensemble_step(e, sink, keep_nut, h);
                 if (rc && h == hipSuccess) h = hipErrorUnknown;
             }
             hipError_t h2 = hipStreamEndCapture(e->stream, &g);

@@ -3,7 +3,7 @@ the same bits as steps one call at a time, for the ways a step is launched."""
 import numpy as np
 import pytest
 
-from channel_rl_amd import FP32_BULK, FP64, NU_T, U, V, W, Channel
+from channel_rl_amd import FP32_BULK, FP64, NU_T, U, V, W, Channel, Ensemble
 from test_gpu_parity import cases
 
 pytestmark = pytest.mark.gpu
@@ -30,6 +30,34 @@ def test_nu_t_after_several_steps(gpu, monkeypatch, mass, limit, graph, precisio
             g.run_steps(n)
         got.append([g.get_field(w) for w in (NU_T, U, V, W)])
         g.close()
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+# the same of an ensemble: two grouped members and a lone one
+@pytest.mark.parametrize("precision", [FP64, FP32_BULK])
+def test_nu_t_after_several_ensemble_steps(gpu, precision):
+    got = []
+    for calls in ([5], [1] * 5, [3, 2]):
+        chans = []
+        for n, seed in (((34, 17, 26), 3), ((34, 17, 26), 4), ((18, 9, 10), 5)):
+            case, field = cases.small_case(*n, seed=seed)
+            g = Channel(case.x, case.y, case.z, precision=precision, **dict(case.kwargs(), x_mass_cte=2))
+            g.set_state(*field)
+            g.apply_boundary_conditions()
+            g.compute_projection_step()
+            g.set_scalars(dt=0.0, t=0.0, dPdx=case.dPdx)
+            g.initialize_mass_flow()
+            g.set_wall_model(1, h_wm=case.h_wm)
+            chans.append(g)
+        e = Ensemble(chans)
+        assert e.group_count() == 2
+        for n in calls:
+            e.run_steps(n)
+        got.append([g.get_field(w) for g in chans for w in (NU_T, U, V, W)])
+        e.close()
+        [g.close() for g in chans]
     for other in got[1:]:
         for a, b in zip(got[0], other):
             assert np.isfinite(a).all() and np.array_equal(a, b)
