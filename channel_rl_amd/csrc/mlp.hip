@@ -607,13 +607,15 @@ __global__ void k_wm_samples(const T* U, const T* W, const double* alpha, const 
 // log law's (u_tau^2, 0) by more than max_err relative to u_tau^2; then the
 // equilibrium value.  Writes alpha_x and, per 16-cell group, the sum of
 // relative errors and the number of fallbacks.
-// A wave takes 64 cells at a time, one per lane: each lane samples the flow
-// and forms the features of its own cell, the network runs on the four
+// A wave takes 16 nq cells at a time, one per lane: each lane samples the flow
+// and forms the features of its own cell, the network runs on the nq (1, 2, 4)
 // 16-cell groups in turn (an MFMA pass takes 16 samples, the features of
 // group q broadcast from lanes 16q..16q+15), and each lane keeps the outputs
-// of its own cell for the FP64 closure that follows.
+// of its own cell for the FP64 closure that follows.  The first cells are
+// sampled while the network's image arrives.
 template <typename T, bool G>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_wm_mlp(WmArgs<T> one, const WmArgs<T>* tab, Dims d)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_wm_mlp(WmArgs<T> one, const WmArgs<T>* tab, Dims d,
+                                                                                                  int nq)
 {
     const GBlk gb = gblk(1);
     const WmArgs<T> arg = member_args<G>(one, tab, gb.m);
@@ -626,28 +628,38 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     const int x_mass_cte = arg.x_mass_cte;
     __shared__ MlpNet s;
     mlp_copy_image(s, static_cast<const MlpNet*>(arg.net));
-    __syncthreads();
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     const long ncell = 2L * d.nx * d.nzg;
     const long ngroups = (ncell + 15) / 16;
-    const long nquad = (ncell + 63) / 64;
+    const int per = 16 * nq;  // cells a wave takes at a time
+    const long nset = (ncell + per - 1) / per;
     const double dpdx = wm_driving_dpdx(sc, x_mass_cte);
-    for (long qd = (long)gb.x * 4 + wave; qd < nquad; qd += (long)gb.gx * 4) {
-        lds_reload_fence();
-        const long c = qd * 64 + lane;
-        const bool ok = c < ncell;
-        float xo[4] = {0.f, 0.f, 0.f, 0.f};
-        WallSample ws{0.0, 0.0, 0.0, 1.0};
+    WallSample ws;
+    float f[4];
+    bool ok;
+    auto sample = [&](long set) {
+        const long c = set * per + lane;
+        ok = lane < per && c < ncell;
+        ws = WallSample{0.0, 0.0, 0.0, 1.0};
+        for (int q = 0; q < 4; q++) f[q] = 0.f;
         if (ok) {
             const int i = (int)(c % d.nx) + 1, wall = (int)((c / d.nx) % 2), k = (int)(c / (2L * d.nx)) + 1;
             ws = wall_sample(U, W, m, d, i, k, wall, h_wm);
-            float f[4];
             wm_features(ws, nu, alpha[c], dpdx, f);
-            for (int q = 0; q < 4; q++) xo[q] = (f[q] - s.xm[q]) / s.xs[q];
         }
+    };
+    long set = (long)gb.x * 4 + wave;
+    sample(set);
+    __syncthreads();
+    for (; set < nset; set += (long)gb.gx * 4, sample(set)) {
+        lds_reload_fence();
+        const long c = set * per + lane;
+        float xo[4] = {0.f, 0.f, 0.f, 0.f};
+        if (ok)
+            for (int q = 0; q < 4; q++) xo[q] = (f[q] - s.xm[q]) / s.xs[q];
         float ys[2] = {0.f, 0.f};
 #pragma unroll 1
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < nq; q++) {
             lds_reload_fence();
             float x[4];
             for (int e = 0; e < 4; e++) x[e] = __shfl(xo[e], 16 * q + lane % 16);
@@ -680,8 +692,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
             err += __shfl_xor(err, o);
             fb += __shfl_xor(fb, o);
         }
-        const long grp = qd * 4 + lane / 16;
-        if (lane % 16 == 0 && grp < ngroups) {
+        const long grp = set * nq + lane / 16;
+        if (lane % 16 == 0 && lane < per && grp < ngroups) {
             stats[grp] = err;
             stats[ngroups + grp] = fb;
         }
@@ -710,17 +722,24 @@ void launch_wm_samples(const T* U, const T* W, const double* alpha, const Scalar
 
 long wm_mlp_groups(const Dims& d) { return (2L * d.nx * d.nzg + 15) / 16; }
 
-// blocks of 4 waves, one 64-cell set per wave: a set's forward passes take
+// Blocks of 4 waves, one set of cells per wave: a set's forward passes take
 // several microseconds of dependent instructions, so waves rather than
-// loop trips carry the cells (the 18.8 KB image copy per block comes from L2)
+// loop trips carry the cells (the 18.8 KB image copy per block comes from L2).
+// Fewer cells a wave, and so fewer passes in turn, while that leaves about one
+// wave a SIMD; beyond it the FP64 parts, which cost a wave the same for 16
+// cells as for 64, decide.  us with 16 / 32 / 64 cells a wave: 32^2 walls 13.4 /
+// 13.8 / 18.0, 64^2 12.7 / 14.6 / 18.8, 96^2 17.8 / 16.9 / 20.9, 128^2 22.5 / 20.5
+// / 21.4, 192^2 32.8 / 26.5 / 26.4, a group of 27 of 96^2 189 / 121 / 90.
 template <typename T>
 void run_wm_mlp(const WmArgs<T>& one, const WmArgs<T>* tab, int nmem, const Dims& d, hipStream_t s)
 {
-    const long quads = (2L * d.nx * d.nzg + 63) / 64;
-    const int blocks = (int)std::max(1L, std::min(2048L, (quads + 3) / 4));
+    const long cells = 2L * d.nx * d.nzg;
+    const int nq = cells * nmem <= 16 * 1200 ? 1 : (cells * nmem <= 32 * 1200 ? 2 : 4);
+    const long sets = (cells + 16 * nq - 1) / (16 * nq);
+    const int blocks = (int)std::max(1L, std::min(2048L, (sets + 3) / 4));
     PROF_BEGIN("k_wm_mlp", s);
-    if (tab) k_wm_mlp<T, true><<<dim3(blocks, 1, nmem), 256, 0, s>>>(one, tab, d);
-    else k_wm_mlp<T, false><<<dim3(blocks, 1, 1), 256, 0, s>>>(one, nullptr, d);
+    if (tab) k_wm_mlp<T, true><<<dim3(blocks, 1, nmem), 256, 0, s>>>(one, tab, d, nq);
+    else k_wm_mlp<T, false><<<dim3(blocks, 1, 1), 256, 0, s>>>(one, nullptr, d, nq);
     PROF_END(s);
 }
 
