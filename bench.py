@@ -46,10 +46,11 @@ ALG_FLOPS = {"k_dsm_fused": 519}
 #              registers between the sweeps): 2
 #   k_fftx_inv: reads p-hat (1), writes p (1)
 #   k_project: reads p, U,V,W, writes U,V,W: 7
-# A whole step of the dynamic model (mass-flow mode 1) moves 107 values per
+# A step of the dynamic model on its own (mass-flow mode 1) moves 107 values per
 # cell (856 B FP64, 548 B FP32 bulk): compute_dt rides in the first pass A,
 # pass B runs in the last substep only (the RHS converts |S| in the others)
-# and the mass-flow shift in the last projection.  step_alg_gbs sums these
+# and the mass-flow shift in the last projection.  Of several steps in a call
+# only the last runs pass B: 105 values in the others.  step_alg_gbs sums these
 # per launch over the launches the profiled steps make.
 ALG_VALUES = {
     "k_rhs_rk": (12, 0),
@@ -379,7 +380,12 @@ def main():
     from channel_rl_amd import rocprof_summary
     tag = f"{case.nx - 2}x{case.ny}x{case.nz - 2}_{args.precision}" + ("_amd" if args.les == "amd" else "")
     traffic_all = rocprof_summary.load_traffic(os.path.join(ROOT, "profiles", f"hbm_traffic_channel_step_{tag}.md"))
-    traffic = traffic_all.get(dom)
+    def hbm_bytes(name):
+        # the profiles name a stage's kernel by its form: k_tridiag_tw (rows in
+        # registers), k_dsm_fused_fp32 (pass A in FP32)
+        return next((traffic_all[k] for k in (name, name + "_tw", name + "_fp32") if k in traffic_all), None)
+
+    traffic = hbm_bytes(dom)
     # every stage of the step: HIP-event time per launch, algorithmic bytes
     # (where counted) and the HBM bytes of the counter passes, each as a
     # rate and as a fraction of the HBM peak
@@ -396,8 +402,7 @@ def main():
             ab = cells * (b0 * bulk_b + b1 * 8)
             st["alg_bytes"] = ab
             st["alg_hbm_frac"] = round(ab / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)
-        # the profiles name the tridiagonal kernels by their form (k_tridiag_tw: rows in registers)
-        tb = traffic_all.get(name, traffic_all.get(name + "_tw"))
+        tb = hbm_bytes(name)
         if tb is not None:
             st["hbm_bytes"] = int(tb)
             st["hbm_frac"] = round(tb / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)

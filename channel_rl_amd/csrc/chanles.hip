@@ -1256,11 +1256,12 @@ int chan_profile_steps(chan_ctx* c, int nsteps)
     for (int n = 0; n < nsteps && rc == CHAN_OK; n++) {
         if (fuse) {
             rc = net_order(c);
-            if (!rc) rc = DISPATCH(c, rk3_step, c, true, true);
+            if (!rc) rc = DISPATCH(c, rk3_step, c, true, n + 1 == nsteps);
         } else {
             DISPATCH(c, enqueue_dt, c);
             rc = check_launch(c);
-            if (!rc) rc = chan_compute_time_step_RK3(c);
+            if (!rc) rc = net_order(c);
+            if (!rc) rc = DISPATCH(c, rk3_step, c, false, n + 1 == nsteps);
         }
         hipError_t e = hipStreamSynchronize(c->stream);
         if (!rc && e != hipSuccess) rc = fail(c, CHAN_EHIP, std::string("profile sync: ") + hipGetErrorString(e));
