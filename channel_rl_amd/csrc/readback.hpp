@@ -61,9 +61,20 @@ class Readback {
             return true;
         }
     };
-    std::mutex use_;  // held by the copy that uses the slots, and to change the count
+    std::mutex use_;  // held by the copy that uses the slots, never for work before it
     std::unique_ptr<Slots> slots_;
+    std::mutex count_;  // held to change the number of channels
     int channels_ = 0;
+
+    // the slots for a copy from `device` (use_ held), made by the first one
+    bool ready(int device)
+    {
+        if (!slots_) {
+            auto s = std::make_unique<Slots>();
+            if (s->make(device)) slots_ = std::move(s);
+        }
+        return slots_ && slots_->device == device;
+    }
 
     // worker w's chunks w, w + n, ...: one in flight while the one before is copied
     static hipError_t work(Slots& s, int w, int n, char* dst, const char* src, size_t bytes, hipStream_t st)
@@ -98,13 +109,15 @@ public:
     }
     void add_channel()
     {
-        std::lock_guard<std::mutex> l(use_);
+        std::lock_guard<std::mutex> l(count_);
         channels_++;
     }
     void remove_channel()
     {
-        std::lock_guard<std::mutex> l(use_);
-        if (--channels_ == 0) slots_.reset();
+        std::lock_guard<std::mutex> l(count_);
+        if (--channels_ > 0) return;
+        std::lock_guard<std::mutex> u(use_);  // free: a copy needs a channel
+        slots_.reset();
     }
     // src (device memory of `device`, written by earlier work of st) to dst;
     // returns with the copy complete
@@ -113,12 +126,15 @@ public:
         if (bytes >= LEAST && !pinned(dst)) {
             std::unique_lock<std::mutex> l(use_, std::try_to_lock);
             if (l.owns_lock()) {
-                if (!slots_) {
-                    auto s = std::make_unique<Slots>();
-                    if (s->make(device)) slots_ = std::move(s);
-                }
-                if (slots_ && slots_->device == device) return shared(dst, src, bytes, st);
+                (void)ready(device);  // their allocation beside the stream's work
+                l.unlock();
             }
+            // the work before the copy is waited for by this thread alone and
+            // without the slots, which other channels may want meanwhile
+            const hipError_t e = hipStreamSynchronize(st);
+            if (e != hipSuccess) return e;
+            if (l.try_lock() && ready(device)) return shared(dst, src, bytes, st);
+            if (l.owns_lock()) l.unlock();
         }
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
         return e != hipSuccess ? e : hipStreamSynchronize(st);
