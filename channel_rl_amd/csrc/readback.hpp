@@ -123,7 +123,7 @@ public:
     // returns with the copy complete
     hipError_t copy(void* dst, const void* src, size_t bytes, int device, hipStream_t st)
     {
-        if (bytes >= LEAST && !pinned(dst)) {
+        if (bytes >= LEAST && pageable(dst)) {
             std::unique_lock<std::mutex> l(use_, std::try_to_lock);
             if (l.owns_lock()) {
                 (void)ready(device);  // their allocation beside the stream's work
@@ -141,15 +141,16 @@ public:
     }
 
 private:
-    // memory of hipHostMalloc: the runtime's copy is already at the link's rate
-    static bool pinned(const void* p)
+    // memory the runtime does not know; what it knows it copies to itself, at the
+    // link's rate into pinned memory, and a device's the threads cannot write
+    static bool pageable(const void* p)
     {
         hipPointerAttribute_t a{};
         if (hipPointerGetAttributes(&a, p) != hipSuccess) {
             (void)hipGetLastError();
-            return false;
+            return true;
         }
-        return a.type == hipMemoryTypeHost;
+        return a.type == hipMemoryTypeUnregistered;
     }
     hipError_t shared(void* dst, const void* src, size_t bytes, hipStream_t st)
     {

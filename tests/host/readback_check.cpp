@@ -54,9 +54,30 @@ static int busy()
                : 1;
 }
 
+// Memory that the runtime knows (the device's, managed, pinned) is copied by one
+// call of the runtime: the copy's threads could not write the device's.
+static int known()
+{
+    Readback& r = Readback::get();
+    r.add_channel();
+    const std::vector<char> src = pattern(3);
+    int bad = 0;
+    for (int type : {hipMemoryTypeDevice, hipMemoryTypeManaged, hipMemoryTypeHost}) {
+        fake_type = type;
+        std::vector<char> dst(BYTES);
+        FakeStream s;
+        const hipError_t e = r.copy(dst.data(), src.data(), BYTES, 0, &s);
+        std::printf("type %d: %d copies, the largest of %zu bytes\n", type, s.copies.load(), s.largest.load());
+        bad += e != hipSuccess || dst != src || s.copies != 1 || s.largest != BYTES;
+    }
+    r.remove_channel();
+    return bad;
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "busy") return busy();
+    if (what == "known") return known();
     return 2;
 }
