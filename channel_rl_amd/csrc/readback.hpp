@@ -8,8 +8,8 @@
 #include <exception>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
-#include <vector>
 
 namespace chan {
 
@@ -70,8 +70,8 @@ class Readback {
     bool ready(int device)
     {
         if (!slots_) {
-            auto s = std::make_unique<Slots>();
-            if (s->make(device)) slots_ = std::move(s);
+            std::unique_ptr<Slots> s(new (std::nothrow) Slots);
+            if (s && s->make(device)) slots_ = std::move(s);
         }
         return slots_ && slots_->device == device;
     }
@@ -104,7 +104,9 @@ class Readback {
 public:
     static Readback& get()
     {
-        static Readback* const r = new Readback;  // outlives the runtime's own teardown
+        // never destroyed: it outlives the runtime's own teardown
+        alignas(Readback) static unsigned char mem[sizeof(Readback)];
+        static Readback* const r = ::new (mem) Readback;
         return *r;
     }
     void add_channel()
@@ -157,16 +159,15 @@ private:
         const int n = (int)std::min<size_t>(WORKERS, (bytes + 2 * CHUNK - 1) / (2 * CHUNK));
         hipError_t res[WORKERS] = {};
         auto part = [&](int w) { res[w] = work(*slots_, w, n, (char*)dst, (const char*)src, bytes, st); };
-        std::vector<std::thread> t;
-        t.reserve(WORKERS);
+        std::thread t[WORKERS];
         int made = 1;  // this thread takes part 0, and those that got no thread
         try {
-            for (; made < n; made++) t.emplace_back(part, made);
+            for (; made < n; made++) t[made] = std::thread(part, made);
         } catch (const std::exception&) {
         }
         part(0);
         for (int w = made; w < n; w++) part(w);
-        for (auto& x : t) x.join();
+        for (int w = 1; w < made; w++) t[w].join();
         // nothing of this copy is left in flight when the slots go to the next
         hipError_t e = hipStreamSynchronize(st);
         for (int w = 0; w < n; w++)

@@ -8,7 +8,6 @@
 #include <cstddef>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
 #include <mutex>
 #include <vector>
 
@@ -24,14 +23,15 @@ struct FakeStream {
     bool open = true;
     std::atomic<int> waiting{0}, copies{0};
     std::atomic<size_t> largest{0};
-    std::vector<std::function<void()>> queue;
+    struct Copy { void* d; const void* s; size_t n; };
+    std::vector<Copy> queue;
     void wait()
     {
         std::unique_lock<std::mutex> l(mu);
         waiting++;
         cv.wait(l, [&] { return open; });
         waiting--;
-        for (auto& f : queue) f();
+        for (const Copy& c : queue) std::memcpy(c.d, c.s, c.n);
         queue.clear();
     }
     void gate(bool o)
@@ -90,7 +90,7 @@ inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind
     std::lock_guard<std::mutex> l(st->mu);
     st->copies++;
     if (n > st->largest) st->largest = n;
-    st->queue.push_back([=] { std::memcpy(d, s, n); });
+    st->queue.push_back({d, s, n});
     return hipSuccess;
 }
 inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*)

@@ -5,10 +5,28 @@
 #include <chrono>
 #include <cstdio>
 #include <future>
+#include <new>
 #include <string>
 
 using chan::Readback;
 using namespace std::chrono_literals;
+
+// from here on this many allocations succeed and the rest fail (below 0: all succeed)
+static std::atomic<int> fake_budget{-1};
+static void* fake_new(size_t n)
+{
+    int b = fake_budget;
+    while (b > 0 && !fake_budget.compare_exchange_weak(b, b - 1)) {}
+    return b == 0 ? nullptr : std::malloc(n ? n : 1);
+}
+void* operator new(size_t n)
+{
+    if (void* p = fake_new(n)) return p;
+    throw std::bad_alloc();
+}
+void* operator new(size_t n, const std::nothrow_t&) noexcept { return fake_new(n); }
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 static constexpr size_t BYTES = (37u << 20) + 12345;  // over the threaded copy's limit, a partial last chunk
 
@@ -74,10 +92,37 @@ static int known()
     return bad;
 }
 
+// No host memory for the slots or for any of the threads: the copy still
+// arrives, and nothing is thrown (its caller is a C function).
+static int memory()
+{
+    const std::vector<char> src = pattern(4);
+    for (int budget = 0; budget < 8; budget++) {
+        std::vector<char> dst(BYTES);
+        FakeStream s;
+        s.queue.reserve(64);  // the runtime's own memory is another matter
+        hipError_t e = hipErrorOutOfMemory;
+        fake_budget = budget;
+        try {
+            Readback::get().add_channel();
+            e = Readback::get().copy(dst.data(), src.data(), BYTES, 0, &s);
+            Readback::get().remove_channel();
+        } catch (const std::bad_alloc&) {
+            fake_budget = -1;
+            std::printf("thrown with %d allocations left\n", budget);
+            return 1;
+        }
+        fake_budget = -1;
+        if (e != hipSuccess || dst != src) return 1;
+    }
+    return 0;
+}
+
 int main(int argc, char** argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "busy") return busy();
     if (what == "known") return known();
+    if (what == "memory") return memory();
     return 2;
 }

@@ -18,7 +18,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["busy", "known"])
+@pytest.mark.parametrize("what", ["busy", "known", "memory"])
 def test_readback(check, what):
     r = subprocess.run([check, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
