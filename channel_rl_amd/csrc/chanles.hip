@@ -1545,7 +1545,8 @@ int chan_synchronize(chan_ctx* c)
 // group (another SGS model, a shape of their own) run their own kernels.
 // One ensemble step (every group and lone member a branch between a fork
 // and a join) is captured into a graph; three graphs cover the rotation of
-// the members' state buffers, each with the argument tables of its phase.
+// the members' state buffers, each with the argument tables of its phase,
+// and three more a call's last step where a member defers nu_t.
 struct chan_ensemble {
     std::string err;
     std::vector<chan_ctx*> ch;
@@ -1900,8 +1901,11 @@ int chan_ensemble_run_steps(chan_ensemble* e, int nsteps)
             h = hipStreamWaitEvent(e->stream, mlp_ready(e->ch[q]->net), 0);
         if (h != hipSuccess) return efail(e, CHAN_EHIP, std::string("ensemble order: ") + hipGetErrorString(h));
     }
+    // one form of a step only where nothing is deferred (rk3_step)
+    bool defers = false;
+    for (const chan_ctx* c : e->ch) defers |= c->defer_nut && c->LES_model == 2;
     for (int it = 0; it < nsteps; it++) {
-        const bool keep_nut = it + 1 == nsteps;
+        const bool keep_nut = !defers || it + 1 == nsteps;
         const int o = (int)(e->step % 3) + (keep_nut ? 3 : 0);
         if (!e->graph[o]) {
             // pass 1: the argument tables of this phase, into device memory
