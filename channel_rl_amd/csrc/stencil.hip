@@ -81,6 +81,34 @@ void launch_bc(T* F, const Dims& d, int kind, hipStream_t s)
 // --------------------------------------------------------------- SGS: DSM
 // Pass A (filters, L_ij, M_ij, plane partial sums, |S|) is dsm_fused.hip.
 
+// Values q = 0..n-1 of N arrays (their starts `stride` apart) to take(), value q by
+// lane q % 64, a lane's in the order of q; past the last, that one again and false.
+// Bound by latency: a lane has U values of each array in flight together, 16, or 4
+// or 1 where that covers the rest (more would only repeat the last value, at 0.3 us
+// a launch for 32x32x32).  k_dsm_ratio at 384x192x384 FP64, 2716 partials a row: 23.2
+// us a launch with one value in flight, 9.5 with 8, 8.4 with 16 or 32 (with
+// compute_dt's 1764 maxima 23.3 -> 9.6); 192x96x192 7.4 -> 5.0 (the launch itself:
+// 4.7).
+template <int U, int N, typename F>
+__device__ __forceinline__ void wave_round(const double* p, int stride, int n, int q0, const F& take)
+{
+    double v[U][N];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int c = 0; c < N; c++) v[u][c] = p[(long)c * stride + min(q0 + 64 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++) take(v[u], q0 + 64 * u < n);
+}
+template <int N, typename F>
+__device__ __forceinline__ void wave_values(const double* p, int stride, int n, int t, const F& take)
+{
+    int b = 0;
+    for (; n - b > 256; b += 64 * 16) wave_round<16, N>(p, stride, n, b + t, take);
+    for (; n - b > 64; b += 64 * 4) wave_round<4, N>(p, stride, n, b + t, take);
+    if (n > b) wave_round<1, N>(p, stride, n, b + t, take);
+}
+
 // <L:M>/<M:M> per row: one wave per row, the blocks' partials summed in a
 // fixed order (strided per lane, then a butterfly across the wave), so the
 // result does not depend on scheduling; no LDS and no barrier.  The row
@@ -111,11 +139,11 @@ __global__ void __launch_bounds__(64) k_dsm_ratio(DsmRatioArgs one, const DsmRat
         const double* dp = ar.dtpart;
         const int nb = ar.nblk_dt;
         double m0 = 0.0, m1 = 0.0, m2 = 0.0;
-        for (int q = t; q < nb; q += 64) {
-            m0 = fmax(m0, dp[q]);
-            m1 = fmax(m1, dp[nb + q]);
-            m2 = fmax(m2, dp[2L * nb + q]);
-        }
+        wave_values<3>(dp, nb, nb, t, [&](const double* v, bool) {
+            m0 = fmax(m0, v[0]);
+            m1 = fmax(m1, v[1]);
+            m2 = fmax(m2, v[2]);
+        });
         for (int m = 32; m > 0; m >>= 1) {
             m0 = fmax(m0, __shfl_xor(m0, m, 64));
             m1 = fmax(m1, __shfl_xor(m1, m, 64));
@@ -128,10 +156,11 @@ __global__ void __launch_bounds__(64) k_dsm_ratio(DsmRatioArgs one, const DsmRat
     double* ratio = ar.ratio;
     const int j = g.x + 2;
     double a = 0.0, c = 0.0;
-    for (int q = t; q < nblk; q += 64) {
-        a += part[((long)(j - 1) * 2 + 0) * nblk + q];
-        c += part[((long)(j - 1) * 2 + 1) * nblk + q];
-    }
+    // (values past the last are added as 0, which changes no sum)
+    wave_values<2>(part + (long)(j - 1) * 2 * nblk, nblk, nblk, t, [&](const double* v, bool in) {
+        a += in ? v[0] : 0.0;
+        c += in ? v[1] : 0.0;
+    });
     for (int m = 32; m > 0; m >>= 1) {
         a += __shfl_xor(a, m, 64);
         c += __shfl_xor(c, m, 64);
