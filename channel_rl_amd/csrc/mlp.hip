@@ -153,20 +153,17 @@ __device__ __forceinline__ void mfma_layer(const bf16x8 (*A)[2][64], const Act& 
 }
 
 // Forward pass of one 16-sample group.  x: standardised features of this
-// lane's sample.  z1..z3: pre-activations; h3q: last hidden layer after BF16
-// rounding; y: standardised outputs (every lane of a sample holds them).
+// lane's sample; y: standardised outputs (every lane of a sample holds them).
 template <bool FAST = false>
-__device__ __forceinline__ void mlp_forward(const MlpNet& s, const float x[4], Act& z1, Act& z2, Act& z3, Act& h3q,
-                                            float y[2])
+__device__ __forceinline__ void mlp_forward(const MlpNet& s, const float x[4], float y[2])
 {
     const int lane = threadIdx.x % 64, g = lane / 16;
-    Act h;
+    Act h, z2, z3;
     for (int t = 0; t < 4; t++)
         for (int r = 0; r < 4; r++) {
             const int n = 16 * t + 4 * g + r;
             float z = s.b1[n];
             for (int k = 0; k < 4; k++) z += x[k] * s.w1[k * 64 + n];
-            z1.a[t * 4 + r] = z;
             h.a[t * 4 + r] = silu_sel<FAST>(z);
         }
     mfma_layer(s.fw[0], h, z2, lane);
@@ -180,9 +177,9 @@ __device__ __forceinline__ void mlp_forward(const MlpNet& s, const float x[4], A
     for (int q = 0; q < 16; q++) {
         const int n = 16 * (q / 4) + 4 * g + (q % 4);
         z3.a[q] += s.b3[n];
-        h3q.a[q] = bfr(silu_sel<FAST>(z3.a[q]));
-        y0 += h3q.a[q] * s.w4[n * 2 + 0];
-        y1 += h3q.a[q] * s.w4[n * 2 + 1];
+        const float h3 = bfr(silu_sel<FAST>(z3.a[q]));
+        y0 += h3 * s.w4[n * 2 + 0];
+        y1 += h3 * s.w4[n * 2 + 1];
     }
     // sum over the four lane groups of this sample, in a fixed order
     y0 += __shfl_xor(y0, 16);
@@ -209,9 +206,8 @@ __global__ void __launch_bounds__(256) k_mlp_infer(const MlpNet* __restrict__ im
         const bool ok = smp < n;
         float x[4];
         for (int k = 0; k < 4; k++) x[k] = ok ? (X[(long)smp * 4 + k] - s.xm[k]) / s.xs[k] : 0.f;
-        Act z1, z2, z3, h3q;
         float y[2];
-        mlp_forward(s, x, z1, z2, z3, h3q, y);
+        mlp_forward(s, x, y);
         if (ok && lane < 16) {
             Y[(long)smp * 2 + 0] = y[0] * s.ys[0] + s.ym[0];
             Y[(long)smp * 2 + 1] = y[1] * s.ys[1] + s.ym[1];
@@ -663,9 +659,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
             lds_reload_fence();
             float x[4];
             for (int e = 0; e < 4; e++) x[e] = __shfl(xo[e], 16 * q + lane % 16);
-            Act z1, z2, z3, h3q;
             float y[2];
-            mlp_forward<true>(s, x, z1, z2, z3, h3q, y);
+            mlp_forward<true>(s, x, y);
             if (lane / 16 == q) { ys[0] = y[0]; ys[1] = y[1]; }
         }
         double err = 0.0, fb = 0.0;
