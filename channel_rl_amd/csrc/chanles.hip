@@ -122,8 +122,9 @@ struct chan_ctx {
     // the same steps with compute_dt folded into substep 1 (dt_fused)
     hipGraphExec_t graph_dt[2][3] = {};
     double* dtpart = nullptr;  // the DSM pass's compute_dt maxima, [3][blocks]
-    // substeps 1 and 2 of a step leave the dynamic model's pass B to the RHS
-    // kernel (DsmBufs::ntab): its row coefficients, [2][nyg] of the bulk type
+    // substeps 1 and 2, and 3 of a step that another follows in the call, leave
+    // the dynamic model's pass B to the RHS kernel (DsmBufs::ntab): its row
+    // coefficients, [2][nyg] of the bulk type
     void* ntab = nullptr;
     bool defer_nut = true;
     double wm_limit = 0.0;  // the wall viscosity limit (a copy of sc->wm_nu_limit)
@@ -1613,7 +1614,8 @@ bool same_group(const chan_ctx* a, const chan_ctx* b)
 {
     return a->prec == b->prec && a->d.nx == b->d.nx && a->d.ny == b->d.ny && a->d.nz == b->d.nz &&
            a->LES_model == 2 && b->LES_model == 2 && a->wall_mode == b->wall_mode && a->x_mass_cte == b->x_mass_cte &&
-           a->rhs_shape == b->rhs_shape && a->dsm_run.tile == b->dsm_run.tile && a->nblk_red == b->nblk_red && a->pb.bx == b->pb.bx && a->pb.bz == b->pb.bz;
+           a->rhs_shape == b->rhs_shape && a->dsm_run.tile == b->dsm_run.tile && a->nblk_red == b->nblk_red &&
+           a->pb.bx == b->pb.bx && a->pb.bz == b->pb.bz;
 }
 
 template <typename T>

@@ -69,8 +69,8 @@ __global__ void __launch_bounds__((TXO + 2) * (TYO + 2)) __attribute__((amdgpu_w
     k_dsm_fused_fp32(DsmArgs<T> one, const DsmArgs<T>* tab, Dims d, int kchunk)
 {
     // The model's sums are reordered against the reference anyway (separable
-    // filter, per-row partials); contracting a*b+c into FMAs here saves a
-    // third of the FP64 instructions and changes results only by rounding.
+    // filter, per-row partials); contracting a*b+c into FMAs here saves
+    // instructions and changes results only by rounding.
 #pragma clang fp contract(fast)
     using Tl = Dsm32<TXO, TYO>;
     constexpr int CX = Tl::CX, NC = Tl::NC, LX = Tl::LX, NL = Tl::NL;

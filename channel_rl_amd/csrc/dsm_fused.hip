@@ -27,12 +27,13 @@
 // reciprocals.  The sums run in a different order than the reference, so the
 // model agrees with it to rounding, not bit for bit.
 // Global traffic: U,V,W read once per tile (plus halo), |S| written once.
-// Measured (192x97x192): 102-112 us a launch against 140-148 before, when every
-// operand of the strains and filters was read from LDS (130 LDS operations and
-// 568 vector instructions a column and plane; now about 60 and 400) from three
-// velocity planes kept there.  Bound by neither LDS (48% busy) nor the FP64
-// units (59%) but by the chain of a plane: two waves per SIMD, all the registers
-// allow, take a plane in 2.3 us where one alone takes 1.2.
+// Measured (192x96x192): 106 us a launch against 142 before, when every operand of
+// the strains and filters was read from LDS, from three velocity planes kept there:
+// a wave's march of 40 planes issued 20,600 vector and 3,700 LDS instructions, now
+// 17,700 and 2,100.  Bound by neither LDS (30% busy, no bank conflicts) nor the
+// vector units (52%) but by the chain of a plane: two waves per SIMD, all the
+// registers allow, take a plane in 2.3 us (106 us less 5 for the launch, over 44
+// planes) where one alone takes 1.2 (12.7 less 3, over 8, at 32x32x32).
 #include <algorithm>
 #include <cmath>
 #include "dsm.hpp"
@@ -256,8 +257,8 @@ __global__ void __launch_bounds__(CX* CY) __attribute__((amdgpu_waves_per_eu(2))
     // strains of those rows either do not use it (V's last row) or are not
     // used (the wall ghost rows); rows further out are clamped and not used.
     auto row = [&](int j, int n) { return j == 0 ? 2 : (j == n + 1 ? n - 1 : min(max(j, 1), n)); };
-    // byte offsets within a plane (below 2^31: a plane holds at most an eighth
-    // of the box's 2^31 values), added to the plane's uniform base address
+    // byte offsets within a plane (below 2^32: the box's 2^31 values are in at
+    // least seven planes), added to the plane's uniform base address
     auto bytes = [&](int i, int j) { return (unsigned)(at(d, i, j, 1) * sizeof(double)); };
     auto ld = [&](const double* base, unsigned o) { return *(const double*)((const char*)base + o); };
     unsigned own = bytes(ic, row(cj, d.nyg)), ownv = bytes(ic, row(cj, d.ny));
@@ -337,8 +338,9 @@ __global__ void __launch_bounds__(CX* CY) __attribute__((amdgpu_waves_per_eu(2))
             {
                 // level 1 of this column at plane p: the filter inputs a (3),
                 // a_a a_b (6), |S| S_ij (6).  Rows outside 2..nyg-1 compute on
-                // the zeros loaded there and finite metric factors; they enter
-                // the y taps of rows 2 and nyg-1 only with weight 0.
+                // the mirrored or clamped rows loaded there and finite metric
+                // factors, and are not used: the y taps of rows 2 and nyg-1 read
+                // their inner neighbour for both (qm, qp).
                 double s[6], uL;
                 strain(vel, nxt, mxc, my.r, mz[0][p - kb + 3], mz[2][p - kb + 3], s, uL);
                 const double sm = magnitude(s);
@@ -420,7 +422,7 @@ __global__ void __launch_bounds__(CX* CY) __attribute__((amdgpu_waves_per_eu(2))
                 }
                 // tp holds 216 times the filtered inputs and sh 216 times
                 // hat(S): with r = 1/216, L = r (T_ab - r T_a T_b) and
-                // M = 4 |hat S| hat S_ab - r T(|S| S_ab) = r (4 r |sh| sh_ab - double),
+                // M = 4 |hat S| hat S_ab - r T(|S| S_ab) = r (4 r |sh| sh_ab - T(|S| S_ab)),
                 // the outer factors taken once on the sums
                 const double r = 1.0 / 216.0;
                 const double shm4 = (4.0 * r) * magnitude(sh);
